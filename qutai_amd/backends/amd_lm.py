@@ -450,8 +450,10 @@ def _check_attention(q, k, v, batch, time, heads, kv_heads, dim):
 def attention(q, k, v, batch, time, heads, kv_heads, dim, *, causal=True, layout=1, scale=None):
     """Attention forward (cuda_lm.attention, src/qutai/backends/cuda_lm.py:229-275):
     (out, lse float32).  bf16 q/k/v with head dimension 64 run the fused MFMA
-    kernel; other head dimensions (<= 256) and float32 storage run the
-    one-wave-per-row kernel, as the reference falls back to its warp kernel.
+    kernel; other head dimensions (<= 256) and float32 storage run the MFMA
+    kernels that keep fp32 values in bf16 parts, rows that are not 16-byte
+    aligned (and fp32 above 128) the one-wave-per-row kernel, the reference's
+    own fallback shape.
     layout 1 is the lm layout [batch][time][heads][dim], layout 0 the nn
     layout [batch][heads][time][dim].  The score matrix is never stored."""
     _check_attention(q, k, v, batch, time, heads, kv_heads, dim)

@@ -26,14 +26,10 @@
 //    leaves registers;
 //  * O^T's result layout gives every lane one query, so the rescaling by
 //    exp(m_old - m_new) and the final 1/l are per-lane scalars.
-#include "common.h"
-#include "qutai_amd.h"
+#include "attention_common.h"
 
 #include <algorithm>
 #include <cstdlib>
-#include <initializer_list>
-
-using namespace qa;
 
 namespace {
 
@@ -66,17 +62,6 @@ typedef i16x4 __attribute__((address_space(3))) * lds_i16x4;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
   uint32_t n = bytes > 0x7ffffff0 ? 0x7ffffff0u : (uint32_t)bytes;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, 0x00020000);
-}
-
-// Both halves of the wavefront (lanes l and l ^ 32) hold the same query:
-// the gfx950 half swap exchanges them without LDS.
-__device__ __forceinline__ float pair_max(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float pair_sum(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // The 32 keys 32 mb + [0, 32) of a 64-key block for the wave's NQB query
@@ -396,8 +381,6 @@ struct AttnBwdArgs {
   float* part_v;
   int64_t part_stride;
 };
-
-constexpr float LOG2E = 1.4426950408889634f;
 
 // Row-fragment of a [64][64] LDS tile whose 16-byte chunks are swizzled by
 // swz_row8: row r, d = 16 s + 8 half + [0, 8) (A operand with k = d, or B
@@ -896,239 +879,6 @@ __global__ void dkv_reduce(const float* pk, const float* pv, bf16_t* dk, bf16_t*
   }
 }
 
-// ============================================================================
-// Generic path: any head dimension up to 256, fp32 or bf16 storage, fp32
-// math (the reference's warp kernels lm_attention / lm_attention_delta /
-// lm_attention_backward_q / _kv, src/qutai/backends/cuda/lm.cu:65-87 and
-// :289-343, used by cuda_lm for everything but bf16 with D = 64).  One wave
-// per query row (forward, dq) or key row (dk, dv); lane l owns dimensions
-// l, l + 64, l + 128, l + 192; dot products are wave-wide sums.
-// ============================================================================
-
-struct AttnGenArgs {
-  const void* g;
-  const void* q;
-  const void* k;
-  const void* v;
-  const void* o;
-  float* lse;
-  float* delta;
-  void* dq;  // forward: the output
-  void* dk;
-  void* dv;
-  int64_t batch, heads, kv_heads, time, dim;
-  int64_t qb, qh, qt, kb, kh, kt, lb, lh, lt;
-  float scale;
-  int causal;
-};
-
-template <class T> __device__ __forceinline__ float ld(const void* p, int64_t i);
-template <> __device__ __forceinline__ float ld<float>(const void* p, int64_t i) { return ((const float*)p)[i]; }
-template <> __device__ __forceinline__ float ld<bf16_t>(const void* p, int64_t i) {
-  return bf16_to_f32(((const bf16_t*)p)[i]);
-}
-template <class T> __device__ __forceinline__ void st(void* p, int64_t i, float x);
-template <> __device__ __forceinline__ void st<float>(void* p, int64_t i, float x) { ((float*)p)[i] = x; }
-template <> __device__ __forceinline__ void st<bf16_t>(void* p, int64_t i, float x) {
-  ((bf16_t*)p)[i] = f32_to_bf16(x);
-}
-
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int off = 32; off; off >>= 1) x += __shfl_xor(x, off);
-  return x;
-}
-
-constexpr int GEN_WAVES = 4;  // rows per workgroup
-
-// row -> (b, h, t) and its element offset in a q-shaped array
-__device__ __forceinline__ void gen_row(const AttnGenArgs& p, int64_t row, int64_t heads, int64_t& b, int64_t& h,
-                                        int64_t& t) {
-  t = row % p.time;
-  h = (row / p.time) % heads;
-  b = row / (p.time * heads);
-}
-
-template <class T>
-__global__ void __launch_bounds__(GEN_WAVES * 64) attention_fwd_rows(AttnGenArgs p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * GEN_WAVES + (threadIdx.x >> 6);
-  if (row >= p.batch * p.heads * p.time) return;  // whole wave
-  int64_t b, h, t;
-  gen_row(p, row, p.heads, b, h, t);
-  const int64_t kvh = h / (p.heads / p.kv_heads);
-  const int64_t qi = b * p.qb + h * p.qh + t * p.qt, kbase = b * p.kb + kvh * p.kh;
-  const int D = (int)p.dim;
-  float qv[4], acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    qv[j] = d < D ? ld<T>(p.q, qi + d) : 0.f;
-    acc[j] = 0.f;
-  }
-  float m = -INFINITY, l = 0.f;
-  const int64_t end = p.causal ? t + 1 : p.time;
-  for (int64_t s = 0; s < end; s++) {
-    const int64_t ki = kbase + s * p.kt;
-    float dot = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int d = lane + 64 * j;
-      if (d < D) dot += qv[j] * ld<T>(p.k, ki + d);
-    }
-    const float x = wave_sum(dot) * p.scale;
-    const float m_new = fmaxf(m, x);
-    const float alpha = __expf(m - m_new), pr = __expf(x - m_new);
-    l = l * alpha + pr;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int d = lane + 64 * j;
-      acc[j] = acc[j] * alpha + (d < D ? pr * ld<T>(p.v, ki + d) : 0.f);
-    }
-    m = m_new;
-  }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    if (d < D) st<T>(p.dq, qi + d, acc[j] * inv);
-  }
-  if (p.lse && lane == 0) p.lse[b * p.lb + h * p.lh + t * p.lt] = m + __logf(l);
-}
-
-template <class T>
-__global__ void __launch_bounds__(GEN_WAVES * 64) attention_bwd_q_rows(AttnGenArgs p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * GEN_WAVES + (threadIdx.x >> 6);
-  if (row >= p.batch * p.heads * p.time) return;
-  int64_t b, h, t;
-  gen_row(p, row, p.heads, b, h, t);
-  const int64_t kvh = h / (p.heads / p.kv_heads);
-  const int64_t qi = b * p.qb + h * p.qh + t * p.qt, kbase = b * p.kb + kvh * p.kh;
-  const int64_t li = b * p.lb + h * p.lh + t * p.lt;
-  const int D = (int)p.dim;
-  float qv[4], gv[4], acc[4], dl = 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    qv[j] = d < D ? ld<T>(p.q, qi + d) : 0.f;
-    gv[j] = d < D ? ld<T>(p.g, qi + d) : 0.f;
-    dl += d < D ? gv[j] * ld<T>(p.o, qi + d) : 0.f;
-    acc[j] = 0.f;
-  }
-  dl = wave_sum(dl);
-  if (lane == 0) p.delta[li] = dl;
-  const float lse = p.lse[li];
-  const int64_t end = p.causal ? t + 1 : p.time;
-  for (int64_t s = 0; s < end; s++) {
-    const int64_t ki = kbase + s * p.kt;
-    float dot = 0.f, dp = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int d = lane + 64 * j;
-      if (d < D) {
-        dot += qv[j] * ld<T>(p.k, ki + d);
-        dp += gv[j] * ld<T>(p.v, ki + d);
-      }
-    }
-    const float pr = __expf(wave_sum(dot) * p.scale - lse);
-    const float ds = pr * (wave_sum(dp) - dl) * p.scale;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int d = lane + 64 * j;
-      if (d < D) acc[j] += ds * ld<T>(p.k, ki + d);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    if (d < D) st<T>(p.dq, qi + d, acc[j]);
-  }
-}
-
-template <class T>
-__global__ void __launch_bounds__(GEN_WAVES * 64) attention_bwd_kv_rows(AttnGenArgs p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * GEN_WAVES + (threadIdx.x >> 6);
-  if (row >= p.batch * p.kv_heads * p.time) return;
-  int64_t b, kvh, s;
-  gen_row(p, row, p.kv_heads, b, kvh, s);
-  const int64_t ki = b * p.kb + kvh * p.kh + s * p.kt;
-  const int64_t group = p.heads / p.kv_heads;
-  const int D = (int)p.dim;
-  float kv_[4], vv[4], ak[4], av[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    kv_[j] = d < D ? ld<T>(p.k, ki + d) : 0.f;
-    vv[j] = d < D ? ld<T>(p.v, ki + d) : 0.f;
-    ak[j] = av[j] = 0.f;
-  }
-  for (int64_t h = kvh * group; h < (kvh + 1) * group; h++) {
-    for (int64_t t = p.causal ? s : 0; t < p.time; t++) {
-      const int64_t qi = b * p.qb + h * p.qh + t * p.qt;
-      const int64_t li = b * p.lb + h * p.lh + t * p.lt;
-      float dot = 0.f, dp = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int d = lane + 64 * j;
-        if (d < D) {
-          dot += ld<T>(p.q, qi + d) * kv_[j];
-          dp += ld<T>(p.g, qi + d) * vv[j];
-        }
-      }
-      const float pr = __expf(wave_sum(dot) * p.scale - p.lse[li]);
-      const float ds = pr * (wave_sum(dp) - p.delta[li]) * p.scale;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int d = lane + 64 * j;
-        if (d < D) {
-          ak[j] += ds * ld<T>(p.q, qi + d);
-          av[j] += pr * ld<T>(p.g, qi + d);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int d = lane + 64 * j;
-    if (d < D) {
-      st<T>(p.dk, ki + d, ak[j]);
-      st<T>(p.dv, ki + d, av[j]);
-    }
-  }
-}
-
-}  // namespace
-
-extern "C" {
-
-}  // extern "C"
-
-namespace {
-
-// element strides of (batch, head, token) for q-shaped, kv-shaped and lse arrays
-template <class Args>
-int set_layout(Args& a, int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim, int layout) {
-  if (batch < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || time < 0 || dim <= 0) return QA_EINVAL;
-  if (layout != 0 && layout != 1) return QA_EINVAL;
-  if (time > (1 << 30) / (heads > kv_heads ? heads : kv_heads) / dim) return QA_EINVAL;  // 32-bit element offsets
-  a.batch = batch;
-  a.heads = heads;
-  a.kv_heads = kv_heads;
-  a.time = time;
-  if (layout == 0) {  // [batch][heads][time][dim]
-    a.qb = heads * time * dim, a.qh = time * dim, a.qt = dim;
-    a.kb = kv_heads * time * dim, a.kh = time * dim, a.kt = dim;
-    a.lb = heads * time, a.lh = time, a.lt = 1;
-  } else {            // [batch][time][heads][dim] (the lm layout)
-    a.qb = time * heads * dim, a.qh = dim, a.qt = heads * dim;
-    a.kb = time * kv_heads * dim, a.kh = dim, a.kt = kv_heads * dim;
-    a.lb = time * heads, a.lh = 1, a.lt = heads;
-  }
-  return QA_OK;
-}
-
 // Workgroup shape of every attention kernel: 8 waves (two per SIMD, so one
 // wave's softmax overlaps the other's MFMAs) of 32 queries or keys, or 4
 // waves of 64; QUTAI_AMD_ATTN_WAVES=4|8 overrides the default 8 (tuning).
@@ -1138,18 +888,6 @@ int attention_waves() {
     return v && atoi(v) == 4 ? 4 : 8;
   }();
   return waves;
-}
-
-int64_t cu_count() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 // Workspace of the dK/dV query-head split: with grouped-query attention
@@ -1162,12 +900,6 @@ size_t dkv_split_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t t
   const int64_t blocks_k = batch * kv_heads * ((time + 255) / 256);
   if (blocks_k >= 2 * cu_count()) return 0;
   return (size_t)2 * (heads / kv_heads) * batch * time * kv_heads * D * sizeof(float);
-}
-
-bool aligned16(std::initializer_list<const void*> ptrs) {
-  for (const void* ptr : ptrs)
-    if (!ptr || (uintptr_t)ptr % 16) return false;
-  return true;
 }
 
 }  // namespace
@@ -1201,32 +933,14 @@ int qutai_amd_attention_fwd(const void* q, const void* k, const void* v, void* o
       hipLaunchKernelGGL((attention_fwd_d64<4, 2>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
     return (int)hipGetLastError();
   }
-  if ((dtype != BF16 && dtype != F32) || dim > 256) return QA_EINVAL;
-  AttnGenArgs a = {};
-  if (set_layout(a, batch, heads, kv_heads, time, dim, layout) != QA_OK) return QA_EINVAL;
-  if (batch * time == 0) return QA_OK;
-  a.q = q;
-  a.k = k;
-  a.v = v;
-  a.dq = out;
-  a.lse = lse;
-  a.dim = dim;
-  a.scale = (float)scale;
-  a.causal = causal ? 1 : 0;
-  const int64_t blocks = (batch * heads * time + GEN_WAVES - 1) / GEN_WAVES;
-  if (blocks > 0x7fffffff) return QA_EINVAL;
-  if (dtype == BF16)
-    hipLaunchKernelGGL(attention_fwd_rows<bf16_t>, dim3((unsigned)blocks), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(attention_fwd_rows<float>, dim3((unsigned)blocks), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  return (int)hipGetLastError();
+  return attention_general_fwd(q, k, v, out, lse, batch, heads, kv_heads, time, dim, dtype, layout, scale, causal,
+                               (hipStream_t)stream);
 }
 
 size_t qutai_amd_attention_bwd_workspace_size(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time,
                                               int64_t dim, int dtype) {
-  if (dtype != BF16 || dim != D || batch < 0 || time < 0) return 0;
+  if (dtype != BF16 || dim != D) return attention_general_workspace(batch, heads, kv_heads, time, dim, dtype);
+  if (batch < 0 || time < 0) return 0;
   return dkv_split_bytes(batch, heads, kv_heads, time);
 }
 
@@ -1288,42 +1002,8 @@ int qutai_amd_attention_bwd(const void* grad, const void* q, const void* k, cons
                        (const float*)a.part_v, a.dk, a.dv, n4, a.part_stride, (int)(heads / kv_heads), a.scale);
     return (int)hipGetLastError();
   }
-  if ((dtype != BF16 && dtype != F32) || dim > 256) return QA_EINVAL;
-  AttnGenArgs a = {};
-  if (set_layout(a, batch, heads, kv_heads, time, dim, layout) != QA_OK) return QA_EINVAL;
-  if (batch * time == 0) return QA_OK;
-  a.g = grad;
-  a.q = q;
-  a.k = k;
-  a.v = v;
-  a.o = out;
-  a.lse = const_cast<float*>(lse);
-  a.delta = delta;
-  a.dq = dq;
-  a.dk = dk;
-  a.dv = dv;
-  a.dim = dim;
-  a.scale = (float)scale;
-  a.causal = causal ? 1 : 0;
-  const int64_t blocks_q = (batch * heads * time + GEN_WAVES - 1) / GEN_WAVES;
-  const int64_t blocks_k = (batch * kv_heads * time + GEN_WAVES - 1) / GEN_WAVES;
-  if (blocks_q > 0x7fffffff || blocks_k > 0x7fffffff) return QA_EINVAL;
-  // the q pass writes delta, which the kv pass reads
-  if (dtype == BF16)
-    hipLaunchKernelGGL(attention_bwd_q_rows<bf16_t>, dim3((unsigned)blocks_q), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(attention_bwd_q_rows<float>, dim3((unsigned)blocks_q), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return (int)e;
-  if (dtype == BF16)
-    hipLaunchKernelGGL(attention_bwd_kv_rows<bf16_t>, dim3((unsigned)blocks_k), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(attention_bwd_kv_rows<float>, dim3((unsigned)blocks_k), dim3(GEN_WAVES * 64), 0,
-                       (hipStream_t)stream, a);
-  return (int)hipGetLastError();
+  return attention_general_bwd(grad, q, k, v, out, lse, dq, dk, dv, delta, workspace, workspace_bytes, batch, heads,
+                               kv_heads, time, dim, dtype, layout, scale, causal, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -1,0 +1,159 @@
+// Attention forward and backward for every head width and storage type but
+// bf16 with D = 64 (attention.hip): on the matrix cores where rows are
+// 16-byte aligned (attention_mma.h), one wave per row otherwise
+// (attention_rows.h).
+#include <algorithm>
+#include <type_traits>
+
+#include "attention_rows.h"
+#include "attention_mma.h"
+
+namespace {
+
+// dK = scale * sum_g part_k[g], dV = sum_g part_v[g] (g in order), one
+// rounding to the storage type; 4 elements per lane and step.
+template <bool F32>
+__global__ void dkv_sum(AttnGenArgs p, int64_t n4, int group) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+    f32x4 sk = global_load<f32x4>(p.part_k + 4 * i), sv = global_load<f32x4>(p.part_v + 4 * i);
+    for (int g = 1; g < group; g++) {
+      sk += global_load<f32x4>(p.part_k + g * p.part_stride + 4 * i);
+      sv += global_load<f32x4>(p.part_v + g * p.part_stride + 4 * i);
+    }
+    put4<F32>(p.dk, 4 * i, sk * p.scale);
+    put4<F32>(p.dv, 4 * i, sv);
+  }
+}
+
+enum Pass { FORWARD, QUERIES, KEYS };
+
+template <bool F32, int DP>
+void launch_pass(Pass pass, const AttnGenArgs& a, unsigned blocks, hipStream_t stream) {
+  const dim3 grid(blocks), block(256);
+  if (pass == FORWARD) hipLaunchKernelGGL((attention_fwd_mma<F32, DP>), grid, block, 0, stream, a);
+  else if (pass == QUERIES) hipLaunchKernelGGL((attention_bwd_dq_mma<F32, DP>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((attention_bwd_dkv_mma<F32, DP>), grid, block, 0, stream, a);
+}
+
+// The kernel width DP is the smallest built one that holds the head
+// dimension: the MFMAs work on whole 32-wide d blocks.  fp32 above 128 would
+// need more registers than a wave has (three parts of q and dO).
+bool mma_fits(int dtype, int64_t dim) { return dtype == BF16 ? dim % 8 == 0 && dim <= 256 : dim % 4 == 0 && dim <= 128; }
+
+hipError_t launch_mma(Pass pass, int dtype, const AttnGenArgs& a, int64_t blocks, hipStream_t stream) {
+  const unsigned n = (unsigned)blocks;
+  if (dtype == BF16) {
+    if (a.dim <= 32) launch_pass<false, 32>(pass, a, n, stream);
+    else if (a.dim <= 96) launch_pass<false, 96>(pass, a, n, stream);
+    else if (a.dim <= 128) launch_pass<false, 128>(pass, a, n, stream);
+    else launch_pass<false, 256>(pass, a, n, stream);
+  } else {
+    if (a.dim <= 32) launch_pass<true, 32>(pass, a, n, stream);
+    else if (a.dim <= 64) launch_pass<true, 64>(pass, a, n, stream);
+    else if (a.dim <= 96) launch_pass<true, 96>(pass, a, n, stream);
+    else launch_pass<true, 128>(pass, a, n, stream);
+  }
+  return hipGetLastError();
+}
+
+template <class Kernel>
+hipError_t launch_rows(Kernel bf16, Kernel fp32, int dtype, const AttnGenArgs& a, int64_t rows, hipStream_t stream) {
+  hipLaunchKernelGGL((dtype == BF16 ? bf16 : fp32), dim3((unsigned)((rows + GEN_WAVES - 1) / GEN_WAVES)),
+                     dim3(GEN_WAVES * 64), 0, stream, a);
+  return hipGetLastError();
+}
+
+void set_scale(AttnGenArgs& a, double scale) {
+  a.scale = (float)scale;
+  a.scale_log2 = (float)(scale * 1.4426950408889634);
+  a.scale_log2_lo = (float)(scale * 1.4426950408889634 - (double)a.scale_log2);
+}
+
+constexpr int64_t OWNED = 128;  // queries or keys of a workgroup
+
+// Partial dK/dV of the query heads of each kv head's group, for grids of
+// fewer workgroups than the GPU holds at once (two per CU).
+size_t split_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim) {
+  if (kv_heads <= 0 || heads <= kv_heads || heads % kv_heads) return 0;
+  if (batch * kv_heads * ((time + OWNED - 1) / OWNED) >= 2 * cu_count()) return 0;
+  return (size_t)2 * (heads / kv_heads) * batch * time * kv_heads * dim * sizeof(float);
+}
+
+}  // namespace
+
+int attention_general_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int64_t batch,
+                          int64_t heads, int64_t kv_heads, int64_t time, int64_t dim, int dtype, int layout,
+                          double scale, int causal, hipStream_t stream) {
+  if ((dtype != BF16 && dtype != F32) || dim > 256) return QA_EINVAL;
+  AttnGenArgs a = {};
+  if (set_layout(a, batch, heads, kv_heads, time, dim, layout) != QA_OK) return QA_EINVAL;
+  if (batch * time == 0) return QA_OK;
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.dq = out;
+  a.lse = lse;
+  a.dim = dim;
+  set_scale(a, scale);
+  a.causal = causal ? 1 : 0;
+  const int64_t rows = batch * heads * time;
+  if ((rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
+  if (mma_fits(dtype, dim) && aligned16({q, k, v, out}))
+    return (int)launch_mma(FORWARD, dtype, a, batch * heads * ((time + OWNED - 1) / OWNED), stream);
+  return (int)launch_rows(attention_fwd_rows<bf16_t>, attention_fwd_rows<float>, dtype, a, rows, stream);
+}
+
+size_t attention_general_workspace(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim,
+                                   int dtype) {
+  if ((dtype != BF16 && dtype != F32) || dim <= 0 || batch < 0 || time < 0 || !mma_fits(dtype, dim)) return 0;
+  return split_bytes(batch, heads, kv_heads, time, dim);
+}
+
+int attention_general_bwd(const void* grad, const void* q, const void* k, const void* v, const void* out,
+                          const float* lse, void* dq, void* dk, void* dv, float* delta, void* workspace,
+                          size_t workspace_bytes, int64_t batch, int64_t heads, int64_t kv_heads, int64_t time,
+                          int64_t dim, int dtype, int layout, double scale, int causal, hipStream_t stream) {
+  if ((dtype != BF16 && dtype != F32) || dim > 256) return QA_EINVAL;
+  AttnGenArgs a = {};
+  if (set_layout(a, batch, heads, kv_heads, time, dim, layout) != QA_OK) return QA_EINVAL;
+  if (batch * time == 0) return QA_OK;
+  a.g = grad;
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.o = out;
+  a.lse = const_cast<float*>(lse);
+  a.delta = delta;
+  a.dq = dq;
+  a.dk = dk;
+  a.dv = dv;
+  a.dim = dim;
+  set_scale(a, scale);
+  a.causal = causal ? 1 : 0;
+  const int64_t q_rows = batch * heads * time, k_rows = batch * kv_heads * time;
+  if ((q_rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
+  // the q pass writes delta, which the kv pass reads
+  if (!mma_fits(dtype, dim) || !aligned16({grad, q, k, v, out, dq, dk, dv})) {
+    const hipError_t e =
+        launch_rows(attention_bwd_q_rows<bf16_t>, attention_bwd_q_rows<float>, dtype, a, q_rows, stream);
+    if (e != hipSuccess) return (int)e;
+    return (int)launch_rows(attention_bwd_kv_rows<bf16_t>, attention_bwd_kv_rows<float>, dtype, a, k_rows, stream);
+  }
+  const int64_t blocks = (time + OWNED - 1) / OWNED, group = heads / kv_heads;
+  const size_t need = split_bytes(batch, heads, kv_heads, time, dim);
+  if (need && workspace && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0) {
+    a.split = 1;
+    a.part_stride = batch * time * kv_heads * dim;
+    a.part_k = (float*)workspace;
+    a.part_v = a.part_k + group * a.part_stride;
+  }
+  hipError_t e = launch_mma(QUERIES, dtype, a, batch * heads * blocks, stream);
+  if (e != hipSuccess) return (int)e;
+  e = launch_mma(KEYS, dtype, a, batch * kv_heads * blocks * (a.split ? group : 1), stream);
+  if (e != hipSuccess || !a.split) return (int)e;
+  const int64_t n4 = a.part_stride / 4;
+  const unsigned grid = (unsigned)std::min<int64_t>((n4 + 255) / 256, 1 << 20);
+  if (dtype == BF16) hipLaunchKernelGGL(dkv_sum<false>, dim3(grid), dim3(256), 0, stream, a, n4, (int)group);
+  else hipLaunchKernelGGL(dkv_sum<true>, dim3(grid), dim3(256), 0, stream, a, n4, (int)group);
+  return (int)hipGetLastError();
+}

@@ -1,0 +1,93 @@
+"""Attention on the matrix cores for every head width and storage type beside
+bf16 with 64 (attention_mma.h) against the float64 oracle, at the edges of its
+tiles: 32 queries or keys per wave, 128 per workgroup, streamed blocks of 32 or
+64, kernel widths 32, 64, 96, 128 and 256.
+
+Tolerances: bf16 storage rounds each result once (2^-9 at most, about 1.7e-3
+in the norm), the bar is 4e-3; fp32 storage sums up to 300 terms of 2^-24 with
+roundings in the scores ahead of them, the bar is 3e-6."""
+import numpy as np
+import pytest
+
+from oracle import reference as ora
+from tests.helpers import download, normal, stored, upload
+
+pytestmark = pytest.mark.gpu
+
+BAR = {"bfloat16": 4e-3, "float32": 3e-6}
+
+
+@pytest.fixture(scope="module")
+def lm():
+    from qutai_amd.backends import amd, amd_lm
+
+    amd.get_runtime()
+    return amd_lm
+
+
+def run(lm, dtype, dims, causal, layout, change=None):
+    """Device results and stored inputs as [batch][heads][time][dim] float64."""
+    batch, time, heads, kv_heads, dim = dims
+    counts = (heads, kv_heads, kv_heads, heads)
+    host = [normal(sum(dims) + i, batch * time * n * dim) for i, n in enumerate(counts)]
+
+    def split(x, n):
+        if layout == 0:
+            return x.reshape(batch, n, time, dim)
+        return x.reshape(batch, time, n, dim).transpose(0, 2, 1, 3)
+
+    if change:
+        change(*(split(x, n) for x, n in zip(host, counts)))
+    q, k, v, g = (upload(x, dtype) for x in host)
+    out, lse = lm.attention(q, k, v, *dims, causal=causal, layout=layout)
+    grads = lm.attention_backward(g, q, k, v, out, lse, *dims, causal=causal, layout=layout)
+    inputs = [split(stored(x, dtype), n) for x, n in zip(host, counts)]
+    results = [split(download(x).astype(np.float64), n) for x, n in zip((out, *grads), (heads, heads, kv_heads, kv_heads))]
+    lse = download(lse).reshape((batch, time, heads) if layout else (batch, heads, time))
+    return inputs, results, lse.transpose(0, 2, 1) if layout else lse
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("dims", [(1, 31, 2, 1, 8), (2, 32, 2, 2, 32), (1, 33, 4, 1, 40), (1, 127, 2, 1, 64),
+                                  (1, 128, 2, 1, 96), (2, 129, 2, 1, 100), (1, 65, 4, 2, 128), (1, 300, 2, 1, 128),
+                                  (1, 97, 2, 1, 136), (1, 160, 1, 1, 256)])
+@pytest.mark.parametrize("causal,layout", [(True, 1), (False, 0), (False, 1)])
+def test_edges_of_tiles_and_widths(lm, dtype, dims, causal, layout):
+    (q, k, v, g), (out, dq, dk, dv), lse = run(lm, dtype, dims, causal, layout)
+    batch, _, heads, kv_heads, _ = dims
+    group = heads // kv_heads
+    for b in range(batch):
+        for kh in range(kv_heads):
+            dk_sum = dv_sum = 0
+            for h in range(kh * group, (kh + 1) * group):
+                o_ref, l_ref = ora.attention_np(q[b, h], k[b, kh], v[b, kh], causal=causal)
+                dq_ref, dk_ref, dv_ref = ora.attention_backward_np(g[b, h], q[b, h], k[b, kh], v[b, kh], o_ref, l_ref,
+                                                                   causal=causal)
+                dk_sum, dv_sum = dk_sum + dk_ref, dv_sum + dv_ref
+                assert ora.rel_frobenius(out[b, h], o_ref) <= BAR[dtype], ("out", b, h)
+                assert np.abs(lse[b, h] - l_ref).max() <= 4e-6, ("lse", b, h)  # a few ulps of the largest scores
+                assert ora.rel_frobenius(dq[b, h], dq_ref) <= BAR[dtype], ("dq", b, h)
+            assert ora.rel_frobenius(dk[b, kh], dk_sum) <= BAR[dtype], ("dk", b, kh)
+            assert ora.rel_frobenius(dv[b, kh], dv_sum) <= BAR[dtype], ("dv", b, kh)
+
+
+@pytest.mark.parametrize("dtype,dim", [("bfloat16", 128), ("float32", 64)])
+def test_infinite_and_nan_operands_stay_where_they_are(lm, dtype, dim):
+    """An infinity in the last value and a NaN in the last key of a causal
+    sequence: every earlier query is what it is without them, bit pattern
+    aside, and the last one is not finite."""
+    def poison(q, k, v, g):
+        v[0, 0, -1, 3] = np.inf
+        k[0, 0, -2, 5] = np.nan
+        q[0, 0, :, 7] = 0
+
+    def clean(q, k, v, g):
+        q[0, 0, :, 7] = 0
+
+    dims = (1, 150, 1, 1, dim)
+    (q, k, v, _), (out, dq, _, _), lse = run(lm, dtype, dims, True, 1, clean)
+    _, (bad_out, bad_dq, _, bad_dv), bad_lse = run(lm, dtype, dims, True, 1, poison)
+    assert ora.rel_frobenius(bad_out[0, 0, :148], out[0, 0, :148]) <= BAR[dtype]
+    assert ora.rel_frobenius(bad_dq[0, 0, :148], dq[0, 0, :148]) <= BAR[dtype]
+    assert np.abs(bad_lse[0, 0, :148] - lse[0, 0, :148]).max() <= 4e-6
+    assert np.isnan(bad_out[0, 0, 148:]).all(axis=1).all() and np.isnan(bad_dv[0, 0]).any()
