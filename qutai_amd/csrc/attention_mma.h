@@ -37,28 +37,6 @@
 
 namespace qa {
 
-// N bf16 parts of eight fp32 values, largest first (v = sum of the parts up
-// to 2^(-8 N - 1) of v).
-template <int N>
-__device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8 (&out)[N]) {
-  float r[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) r[e] = v[e];
-#pragma unroll
-  for (int n = 0; n < N; n++) {
-    u32x4 w;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      w[e] = pack_bf16x2(r[2 * e], r[2 * e + 1]);
-      if (n + 1 < N) {
-        r[2 * e] -= __uint_as_float(w[e] << 16);
-        r[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
-      }
-    }
-    out[n] = __builtin_bit_cast(bf16x8, w);
-  }
-}
-
 // acc += A B with operands in NA and NB parts: the terms a_i b_j with
 // first <= i + j < max(NA, NB), smallest first.  Three-part operands keep the
 // terms beside a_0 b_0 in an accumulator of their own (first = 1, then

@@ -48,6 +48,28 @@ __device__ __forceinline__ bf16_t f32_to_bf16(float f) { return (bf16_t)(pack_bf
 __device__ __forceinline__ float sigmoid_f(float v) { return __builtin_amdgcn_rcpf(1.f + __expf(-v)); }
 __device__ __forceinline__ float silu_f(float v) { return v * sigmoid_f(v); }
 
+// N bf16 parts of eight fp32 values, largest first (v = sum of the parts up
+// to 2^(-8 N - 1) of v).
+template <int N>
+__device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8 (&out)[N]) {
+  float r[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) r[e] = v[e];
+#pragma unroll
+  for (int n = 0; n < N; n++) {
+    u32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      w[e] = pack_bf16x2(r[2 * e], r[2 * e + 1]);
+      if (n + 1 < N) {
+        r[2 * e] -= __uint_as_float(w[e] << 16);
+        r[2 * e + 1] -= __uint_as_float(w[e] & 0xffff0000u);
+      }
+    }
+    out[n] = __builtin_bit_cast(bf16x8, w);
+  }
+}
+
 // Store through a global (address space 1) pointer: a generic pointer makes
 // the compiler emit flat stores, which also count against lgkmcnt, so every
 // later wait for an LDS read would wait for the stores as well.

@@ -23,6 +23,13 @@ __global__ void __launch_bounds__(Kern::NT) gemm_entry(GemmArgs p) {
   Kern::run(p, smem);
 }
 
+// fp32 on 128x128 tiles and thin ones: two workgroups per CU, 256 registers
+template <class Kern>
+__global__ void __launch_bounds__(Kern::NT, 2) gemm_entry_two(GemmArgs p) {
+  __shared__ __attribute__((aligned(16))) char smem[Kern::LDS_BYTES];
+  Kern::run(p, smem);
+}
+
 template <class Kern>
 __global__ void __launch_bounds__(Kern::NT) pingpong_entry(GemmArgs p) {
   __shared__ __attribute__((aligned(16))) char smem[Kern::LDS_BYTES];
@@ -329,8 +336,12 @@ __global__ void __launch_bounds__(256, 3) prepare_remainder(PrepareArgs a, Remai
 //   R   : short-K row strips (gemm_short.h): bf16 NT with K <= 64, a 128-row
 //         block of A held in registers, 128-column chunks of B through a
 //         two-slot LDS ring, 128-byte row segments staged through LDS
+//   X   : 128x128, 8 waves 2x4 (64x32 per wave), BK 64 / 32, three- / two-stage
+//         ring: two waves per SIMD where a grid has one such tile per CU
+//   Y, Z: 128x64 and 64x64, 4 waves 2x2, BK 64 / 16, three-stage ring, for
+//         grids that larger tiles would leave to a part of the CUs
 enum Tile { TILE_L8D2, TILE_L8R, TILE_L4D2, TILE_S, TILE_N, TILE_W, TILE_H, TILE_T, TILE_U, TILE_S2, TILE_R, TILE_P,
-            TILE_COUNT };
+            TILE_X, TILE_Y, TILE_Z, TILE_COUNT };
 
 template <bool F32, bool TA, bool TB, int BM, int BN, int WM, int WN, int BK, int ST, bool DMA, bool SWIGLU = false,
           bool GATHER_B = false, bool STREAM_A = false>
@@ -341,7 +352,9 @@ hipError_t launch_cfg(GemmArgs p, hipStream_t stream) {
   int64_t blocks = (int64_t)p.tiles_m * tiles_n * (p.groups ? 1 : p.batch);
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(gemm_entry<Kern>, dim3((unsigned)blocks), dim3(Kern::NT), 0, stream, p);
+  if constexpr (F32 && WM * WN == 4 && BM * BN <= 256 * 64)
+    hipLaunchKernelGGL(gemm_entry_two<Kern>, dim3((unsigned)blocks), dim3(Kern::NT), 0, stream, p);
+  else hipLaunchKernelGGL(gemm_entry<Kern>, dim3((unsigned)blocks), dim3(Kern::NT), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -393,6 +406,9 @@ hipError_t launch_tile(Tile tile, GemmArgs p, hipStream_t stream) {
     case TILE_L4D2: return launch_cfg<F32, TA, TB, 256, 256, 2, 2, KR, 2, true>(p, stream);
     case TILE_S: return launch_cfg<F32, TA, TB, 128, 128, 2, 2, KB, 4, true>(p, stream);
     case TILE_S2: return launch_cfg<F32, TA, TB, 128, 128, 2, 2, KB, 2, true>(p, stream);
+    case TILE_X: return launch_cfg<F32, TA, TB, 128, 128, 2, 4, KR, F32 ? 2 : 3, true>(p, stream);
+    case TILE_Y: return launch_cfg<F32, TA, TB, 128, 64, 2, 2, F32 ? 16 : KR, 3, true>(p, stream);
+    case TILE_Z: return launch_cfg<F32, TA, TB, 64, 64, 2, 2, F32 ? 16 : KR, 3, true>(p, stream);
     case TILE_N:
       // one column tile: every A row is read by one workgroup, streamed
       // (nontemporal copies, K per stage 64 bf16 / 32 fp32 = 128 bytes of a
@@ -449,15 +465,14 @@ int64_t cu_count() {
   return cached[dev];
 }
 
-// Tile choice for an M x N output (batch of them) over K; thin outputs use
-// the 256x64 / 64x256 shapes.  QUTAI_AMD_GEMM_TILE=<L8D2|L8R|L4D2|S|N|W|H|T|U|S2|R>
-// overrides the choice (tuning and tests; R applies only where the short-K
-// strip kernel does, other calls then take L8D2).
+// QUTAI_AMD_GEMM_TILE=<L8D2|L8R|L4D2|S|N|W|H|T|U|S2|R|P|X|Y|Z> overrides the
+// tile choice (tuning and tests; R applies only where the short-K strip kernel
+// does, other calls then take L8D2).
 int forced_tile() {
   static int forced = [] {
     const char* v = getenv("QUTAI_AMD_GEMM_TILE");
     if (!v) return -1;
-    const char* names[TILE_COUNT] = {"L8D2", "L8R", "L4D2", "S", "N", "W", "H", "T", "U", "S2", "R", "P"};
+    const char* names[TILE_COUNT] = {"L8D2", "L8R", "L4D2", "S", "N", "W", "H", "T", "U", "S2", "R", "P", "X", "Y", "Z"};
     for (int i = 0; i < TILE_COUNT; i++)
       if (std::string(v) == names[i]) return i;
     return -1;
@@ -465,51 +480,91 @@ int forced_tile() {
   return forced;
 }
 
-Tile pick_tile(int64_t M, int64_t N, int64_t batch, bool bf16, double* cost);
-
-Tile choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16) {
-  if (forced_tile() >= 0) return (Tile)forced_tile();
-  if (N <= 64) return TILE_N;
-  if (M <= 64) return TILE_W;
-  // K <= 64 (bf16; the attention score product S = Q K^T with K = the head
-  // size) is bound by writing the output: a two-stage ring halves the LDS
-  // of the four-stage one, so four workgroups fit per CU instead of two
-  // (config 3's S product 336 -> 291 us)
-  if (bf16 && K <= 64) return TILE_S2;
-  if (K <= 128) return TILE_S;
-  // Wave-quantisation cost of the large tiles, in units of one full round of
-  // 256x256 tiles over the CUs (per unit of K).  Measured on this GPU (bf16,
-  // 4096^3 and the decoder / ragged shapes): a full round of 256x128 tiles
-  // (one per CU) costs 0.665, a full round of 128x128 tiles (two per CU)
-  // 0.70, and a partial round of at most one 128x128 tile per CU 0.5; a
-  // round of 192x256 / 256x192 tiles (bf16) 0.9; a partial round of the
-  // others costs as much as a full one.  Ties (within 3%) go to 256x128,
-  // then 256x192, 192x256, 256x256.
-  return pick_tile(M, N, batch, bf16, nullptr);
+// What a launch of `units` tiles over K costs, in us: K / 64 steps of the
+// time that the most loaded CU takes for its tiles, plus the first copies and
+// the epilogue of each round.  Measured on this GPU with every tile forced over
+// 25 (bf16) and 19 (fp32) shapes from 8 x 1024 x 1024 to 4096^3, whole and
+// partial rounds; the choice is the fastest tile or within 5% of it on all but
+// two of them.  A CU holds one 256x256, 256x128, 192x256, 256x192 or (bf16)
+// eight-wave 128x128 tile, two four-wave 128x128 or 128x64, three or more
+// 64x64: small tiles cost more per output and win where large ones would leave
+// CUs idle (bf16, 1024^3: 128x128 16.8 us, 64x64 11.1; 2048 x 1024 x 2048 with
+// fp32 output: 29.6 and, 128x64, 23.9; fp32, 512^3: 41 and 21).
+double launch_cost(Tile tile, int64_t units, int64_t K, bool bf16, bool ta) {
+  const int64_t cus = cu_count();
+  const int64_t r = (units + cus - 1) / cus;  // tiles of the most loaded CU
+  const double n = (double)r, pairs = (double)(r / 2), odd = (double)(r % 2);
+  double step, round;
+  int64_t held = 1;
+  switch (tile) {
+    case TILE_H: step = (bf16 ? 1.04 : 6.0) * n, round = 5; break;
+    case TILE_T:
+    case TILE_U: step = bf16 ? 1.40 * n : 10.4 * n, round = 6; break;
+    case TILE_S: step = bf16 ? 1.09 * pairs + 0.78 * odd : 6.2 * pairs + 4.2 * odd, round = 4, held = 2; break;
+    // eight waves: bf16 with an MN-major A pays for its transpose reads
+    case TILE_X: step = bf16 ? (ta ? 0.83 : 0.67) * n : 6.1 * pairs + 3.5 * odd, round = 4, held = bf16 ? 1 : 2; break;
+    case TILE_Y: step = bf16 ? 0.80 * pairs + 0.55 * odd : 4.6 * pairs + 3.2 * odd, round = 3, held = 2; break;
+    case TILE_Z: {
+      const double b[] = {0.39, 0.55, 0.70, 0.97}, f[] = {2.0, 2.35, 3.3, 4.35};
+      step = r <= 4 ? (bf16 ? b : f)[r - 1] : (bf16 ? 0.243 : 1.1) * n;
+      round = 2.5, held = 3;
+      break;
+    }
+    default: step = (bf16 ? 1.56 : 10.4) * n, round = 7; break;
+  }
+  return step * (double)K / 64 + round * (double)((r + held - 1) / held);
 }
 
-// The large-tile choice of choose_tile and its cost (rounds of 256x256 tiles
-// over the CUs, per unit of K).
-Tile pick_tile(int64_t M, int64_t N, int64_t batch, bool bf16, double* cost) {
+int64_t tile_count(Tile tile, int64_t rows, int64_t cols, int64_t batch) {
+  int64_t bm = 256, bn = 256;
+  if (tile == TILE_S || tile == TILE_X) bm = bn = 128;
+  else if (tile == TILE_Y) bm = 128, bn = 64;
+  else if (tile == TILE_Z) bm = bn = 64;
+  else if (tile == TILE_H) bn = 128;
+  else if (tile == TILE_T) bm = 192;
+  else if (tile == TILE_U) bn = 192;
+  else if (tile == TILE_N) bn = 64;
+  else if (tile == TILE_W) bm = 64;
+  return ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn) * batch;
+}
+
+// The cheapest tile of an M x N output (batch of them) over K; the first of
+// this order (large to small: less traffic per product) within 3% of the best.
+Tile pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16, bool ta, double* cost) {
+  static const Tile wide[] = {TILE_H, TILE_U, TILE_T, TILE_L8D2, TILE_X, TILE_S, TILE_Y, TILE_Z};
+  static const Tile narrow[] = {TILE_L8D2, TILE_X, TILE_Z};  // fp32: the others never win
+  const Tile* tiles = bf16 ? wide : narrow;
+  const int count = bf16 ? 8 : 3;
+  double best = 1e30, each[8];
+  for (int i = 0; i < count; i++) {
+    each[i] = launch_cost(tiles[i], tile_count(tiles[i], M, N, batch), K, bf16, ta);
+    best = std::min(best, each[i]);
+  }
+  int pick = 0;
+  while (each[pick] > best * 1.03) pick++;
+  if (cost) *cost = each[pick];
+  return tiles[pick];
+}
+
+Tile choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16, bool ta) {
+  if (forced_tile() >= 0) return (Tile)forced_tile();
   const int64_t cus = cu_count();
-  auto rounds = [cus](int64_t tiles) { return (double)(tiles / cus + (tiles % cus ? 1 : 0)); };
-  const int64_t mt = (M + 255) / 256, nt = (N + 255) / 256, ms = (M + 127) / 128, ns = (N + 127) / 128;
-  const int64_t nl = mt * nt * batch, nh = mt * ns * batch, nsm = ms * ns * batch;
-  const double cost_l = rounds(nl);
-  const double cost_h = 0.665 * rounds(nh);
-  const int64_t rs = nsm % (2 * cus);
-  const double cost_s = 0.70 * (double)(nsm / (2 * cus)) + (rs == 0 ? 0.0 : rs <= cus ? 0.5 : 0.70);
-  const double cost_t = bf16 ? 0.9 * rounds((M + 191) / 192 * nt * batch) : 1e30;
-  const double cost_u = bf16 ? 0.9 * rounds(mt * ((N + 191) / 192) * batch) : 1e30;
-  const double best = std::min({cost_l, cost_h, cost_s, cost_t, cost_u});
-  Tile pick = TILE_S;
-  double chosen = cost_s;
-  if (cost_h <= best * 1.03) pick = TILE_H, chosen = cost_h;
-  else if (cost_u <= best * 1.03) pick = TILE_U, chosen = cost_u;
-  else if (cost_t <= best * 1.03) pick = TILE_T, chosen = cost_t;
-  else if (cost_l <= best * 1.03) pick = TILE_L8D2, chosen = cost_l;
-  if (cost) *cost = chosen;
-  return pick;
+  // Thin outputs whose 256-wide tiles fill the CUs twice: the tile that reads
+  // each row of the long operand once.  Fewer: 64x64, four times the
+  // workgroups (4096 x 1024 x 8 logits: 15.5 us in K chunks, 9.8 whole).
+  if (N <= 64 && tile_count(TILE_N, M, N, batch) >= 2 * cus) return TILE_N;
+  if (M <= 64 && N > 64 && tile_count(TILE_W, M, N, batch) >= 2 * cus) return TILE_W;
+  if (N <= 64 || M <= 64) return TILE_Z;
+  // Short K is bound by writing the output.  K <= 64 (bf16; the attention
+  // score product S = Q K^T with K = the head size): a two-stage ring halves
+  // the LDS of the four-stage one, so four workgroups fit per CU instead of
+  // two (config 3's S product 336 -> 291 us).  Grids of less than one 128x128
+  // tile per CU, or outputs that such tiles would pad by a third, take 64x64.
+  const int64_t small = tile_count(TILE_S, M, N, batch);
+  if (K <= 128 && small > cus && 3 * tile_count(TILE_Z, M, N, batch) >= 9 * small)
+    return bf16 && K <= 64 ? TILE_S2 : bf16 ? TILE_S : TILE_X;
+  if (K <= 128) return TILE_Z;
+  return pick_tile(M, N, K, batch, bf16, ta, nullptr);
 }
 
 // Column remainder: an output N = 256 q + r wide with 0 < r <= 64, whose last
@@ -520,14 +575,14 @@ Tile pick_tile(int64_t M, int64_t N, int64_t batch, bool bf16, double* cost) {
 // round).  Returns the first launch's width, or 0 for one launch.  Each
 // output element still sums K through the same MFMA chain (split K sums its
 // chunks in order), so results stay bit-repeatable.
-int64_t column_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16) {
+int64_t column_split(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16, bool ta) {
   if (forced_tile() >= 0 || batch != 1 || M <= 64 || K <= 128 || N < 512) return 0;
   const int64_t r = N % 256;
   if (r == 0 || r > 64) return 0;
   double full = 0.0, main = 0.0;
-  pick_tile(M, N, 1, bf16, &full);
-  pick_tile(M, N - r, 1, bf16, &main);
-  return main + 0.3 < full * 0.97 ? N - r : 0;
+  pick_tile(M, N, K, 1, bf16, ta, &full);
+  pick_tile(M, N - r, K, 1, bf16, ta, &main);
+  return main + 0.3 * launch_cost(TILE_L8D2, 1, K, bf16, ta) < full * 0.97 ? N - r : 0;
 }
 
 // Split-K for plain products whose tiles fill at most a quarter of the CU
@@ -544,80 +599,68 @@ size_t split_bytes(int64_t rows, int64_t cols, int64_t batch, int splits) {
 int tile_rows(Tile tile) {
   switch (tile) {
     case TILE_S:
+    case TILE_X:
+    case TILE_Y:
     case TILE_S2: return 128;
     case TILE_T: return 192;
+    case TILE_Z:
     case TILE_W: return 64;
     default: return 256;
   }
 }
 
-// Tile of a grouped (per-expert rows) launch: 256x64 for thin outputs, else
-// 256x256 or, for bf16, 256x192 when that takes fewer weighted rounds over
-// the CUs (a round of 256x192 tiles costs 0.9 of a 256x256 one, as in
-// choose_tile).  The M tile count is estimated as ceil(rows / 256) plus half
-// a partial tile per group.  The 256x128 / 128x128 tiles measured slower on
-// config 5's experts and are not considered.  Config 5's down product
-// (cols 2048): 256x192 109 us against 123 us for 256x256.
-Tile grouped_tile(int64_t rows, int64_t cols, int groups, bool bf16) {
+// Tile of a grouped (per-expert rows) launch, the M tile count estimated as
+// ceil(rows / tile rows) plus half a partial tile per group: 256x64 for thin
+// outputs of many rows; 256x256 or 256x192 (bf16) where these fill the CUs
+// (config 5's down product, cols 2048: 256x192 109 us against 123 us for
+// 256x256; 256x128 and 128x128 measured slower there); eight-wave 128x128 or
+// 64x64 tiles where a few hundred rows over many experts would leave most of
+// the CUs idle or a 256-row tile mostly empty.
+Tile grouped_tile(int64_t rows, int64_t inner, int64_t cols, int groups, bool bf16) {
   if (forced_tile() >= 0) return (Tile)forced_tile();
-  if (cols <= 64) return TILE_N;
-  if (!bf16) return TILE_L8D2;
-  const int64_t cus = cu_count();
-  auto rounds = [cus](int64_t tiles) { return (double)(tiles / cus + (tiles % cus ? 1 : 0)); };
-  const int64_t tiles_m = (rows + 255) / 256 + groups / 2;
-  const double cost_l = rounds(tiles_m * ((cols + 255) / 256));
-  const double cost_u = 0.9 * rounds(tiles_m * ((cols + 191) / 192));
-  return cost_u < cost_l * 0.97 ? TILE_U : TILE_L8D2;
+  if (cols <= 64) return rows >= 512 * cu_count() ? TILE_N : TILE_Z;
+  Tile pick = TILE_L8D2;
+  double best = 1e30;
+  for (Tile t : {TILE_L8D2, TILE_U, TILE_X, TILE_Z}) {
+    if (!bf16 && t == TILE_U) continue;
+    const int64_t bm = tile_rows(t), tiles_m = (rows + bm - 1) / bm + groups / 2;
+    const double cost = launch_cost(t, tiles_m * tile_count(t, 1, cols, 1), inner, bf16, false);
+    if (cost < best * 0.97) best = cost, pick = t;
+  }
+  return pick;
 }
 
-int64_t tile_count(Tile tile, int64_t rows, int64_t cols, int64_t batch) {
-  int64_t bm = 256, bn = 256;
-  if (tile == TILE_S) bm = bn = 128;
-  else if (tile == TILE_H) bn = 128;
-  else if (tile == TILE_T) bm = 192;
-  else if (tile == TILE_U) bn = 192;
-  else if (tile == TILE_N) bn = 64;
-  else if (tile == TILE_W) bm = 64;
-  return ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn) * batch;
-}
-
-// A plain product whose tiles fill at most a quarter of the tile slots over
-// K >= 4096 splits K.  For bf16 the tile and the split count are then chosen
-// together: each candidate (256x256, 256x128, 128x128) takes the most chunks
-// that fit its slots, at most 8 and at least 1024 of K each, and is priced as
-// its rounds of tiles over the chunk (the wave-quantisation costs of
-// choose_tile, a full 256x256 round being 113 us per 4096 of K on this GPU)
-// plus the partial sums' HBM traffic (s writes, s reads and one output write
-// of rows x cols fp32 at 5 TB/s).  Measured: the decoder head's dX (1024 x
-// 2048 outputs, K = 32768) takes 256x256 in 8 chunks, 158 -> 137 us; the
-// K/V projections' weight gradients (512 x 2048, K = 4096) take 128x128 in
-// 4 chunks, 28 -> 24 us.  The tile may change; a forced tile does not.
-int choose_split(int64_t rows, int64_t cols, int64_t inner, int64_t batch, Tile* tile, bool bf16, int64_t* chunk) {
+// K chunks of a plain product (batch 1): the tile and the chunk count with the
+// lowest launch_cost over one chunk plus the partial sums' traffic ((2 s + 1)
+// x rows x cols fp32 values at 5 TB/s) and 4 us for the launch that adds them
+// up, if that is at least 15% below the product in one piece; below K = 512
+// the second launch and its workspace cost the host more than the GPU gains.  Which products try:
+//  * fp32 and thin outputs (<= 64 columns or rows): every one; their tiles are
+//    long (fp32) or few (512 x 4096 x 512 fp32, K 4096: 128 us in one piece,
+//    32 in eight; a router's 8 logits; 30 x 2048 x 300 bf16: 17 -> 14 us);
+//  * other bf16 products: K >= 4096 over at most a quarter of the 128x128
+//    tile slots (the decoder head's dX, 1024 x 2048 outputs over K = 32768:
+//    158 -> 129 us with 256x256 tiles in 8 chunks); with shorter K the chunks
+//    measured slower.
+int choose_split(int64_t rows, int64_t cols, int64_t inner, int64_t batch, Tile* tile, bool bf16, bool ta,
+                 int64_t* chunk) {
   const int64_t cus = cu_count();
-  const int64_t tiles = tile_count(*tile, rows, cols, batch);
-  const int64_t slots = (*tile == TILE_S ? 2 : 1) * cus;
+  const bool thin = rows <= 64 || cols <= 64;
   int64_t s = 1;
   const char* forced = getenv("QUTAI_AMD_SPLITK");
   if (forced && atoi(forced) > 0) {
     s = atoi(forced);
-  } else if (batch == 1 && tiles * 4 <= slots && inner >= 4096) {
-    s = std::min<int64_t>(8, slots / tiles);
-    if (bf16 && forced_tile() < 0) {
-      double best = 1e30;
-      for (Tile t : {TILE_L8D2, TILE_H, TILE_S}) {
-        const int64_t n = tile_count(t, rows, cols, 1), per = (t == TILE_S ? 2 : 1) * cus;
-        const int64_t st = std::max<int64_t>(1, std::min<int64_t>({8, per / n, inner / 1024}));
-        const int64_t units = n * st, r = (units + cus - 1) / cus;
-        double rounds;
-        if (t == TILE_L8D2) rounds = (double)r;
-        else if (t == TILE_H) rounds = 0.665 * (double)r;
-        else {
-          const int64_t rs = units % (2 * cus);
-          rounds = 0.70 * (double)(units / (2 * cus)) + (rs == 0 ? 0.0 : rs <= cus ? 0.5 : 0.70);
-        }
-        const double k_chunk = (double)((inner + st - 1) / st);
-        const double reduce_us = st > 1 ? (2.0 * st + 1) * rows * cols * 4 / 5.0e6 : 0.0;
-        const double cost = rounds * k_chunk * (113.0 / 4096) + reduce_us;
+  } else if (batch == 1 && forced_tile() < 0 && inner >= 512 && *tile != TILE_N && *tile != TILE_W &&
+             (!bf16 || thin || (inner >= 4096 && tile_count(TILE_S, rows, cols, 1) * 2 <= cus))) {
+    const double whole = launch_cost(*tile, tile_count(*tile, rows, cols, 1), inner, bf16, ta);
+    double best = 0.85 * whole;
+    for (Tile t : {TILE_L8D2, TILE_H, TILE_X, TILE_S, TILE_Z}) {
+      if ((thin && t != TILE_Z) || (!bf16 && (t == TILE_H || t == TILE_S))) continue;
+      const int64_t n = tile_count(t, rows, cols, 1);
+      for (int64_t st = 2; st <= (thin ? 16 : 8) && inner >= 64 * st; st++) {
+        const int64_t c = ((inner + st - 1) / st + 63) / 64 * 64;
+        if ((inner + c - 1) / c != st || (!thin && c < (bf16 ? 512 : 128))) continue;
+        const double cost = launch_cost(t, n * st, c, bf16, ta) + 4 + (2.0 * st + 1) * rows * cols * 4 / 5.0e6;
         if (cost < best) {
           best = cost;
           *tile = t;
@@ -625,13 +668,6 @@ int choose_split(int64_t rows, int64_t cols, int64_t inner, int64_t batch, Tile*
         }
       }
     }
-  } else if (batch == 1 && (*tile == TILE_N || *tile == TILE_W) && tiles * 4 <= cus && inner >= 512) {
-    // a thin output (<= 64 columns or rows) over a few 256-wide blocks, e.g.
-    // a router's logits or a column remainder: latency-bound tiles, so K
-    // chunks down to 64 (up to 16 of them) put the idle CUs to work
-    // (8192 x 2048 x 8 logits of an 8-expert router: 32 workgroups -> 256;
-    // the last column of 4095 x 1000 x 4097: 16 -> 256)
-    s = std::min<int64_t>({16, cus / tiles, (inner + 63) / 64});
   }
   if (s <= 1 || inner < 128) return 1;
   const int64_t c = ((inner + s - 1) / s + 63) / 64 * 64;
@@ -818,16 +854,16 @@ struct Window {
 // sums), wider remainders on the thin tile.
 int plan_windows(int64_t rows, int64_t inner, int64_t cols, int64_t batch, bool bf16, int transpose_left,
                  Window (&w)[2]) {
-  const int64_t main_cols = inner > 0 ? column_split(rows, cols, inner, batch, bf16) : 0;
+  const int64_t main_cols = inner > 0 ? column_split(rows, cols, inner, batch, bf16, transpose_left) : 0;
   const int count = main_cols ? 2 : 1;
   for (int i = 0; i < count; i++) {
     Window& x = w[i];
     x.c0 = i == 0 ? 0 : main_cols;
     x.n = count == 1 ? cols : i == 0 ? main_cols : cols - main_cols;
     x.rows_kernel = i == 1 && x.n <= 8 && !transpose_left;
-    x.tile = choose_tile(rows, x.n, inner, batch, bf16);
+    x.tile = choose_tile(rows, x.n, inner, batch, bf16, transpose_left);
     x.chunk = 0;
-    x.splits = inner > 0 && !x.rows_kernel ? choose_split(rows, x.n, inner, batch, &x.tile, bf16, &x.chunk) : 1;
+    x.splits = inner > 0 && !x.rows_kernel ? choose_split(rows, x.n, inner, batch, &x.tile, bf16, transpose_left, &x.chunk) : 1;
     x.partial = x.splits > 1 ? split_bytes(rows, x.n, batch, x.splits) : 0;
 
   }
@@ -1044,7 +1080,7 @@ int qutai_amd_gemm_grouped(const void* a, const void* b, void* out, const int64_
     p.a_rows = gather;
     p.a_bytes = source_rows * inner * es;
   }
-  Tile tile = grouped_tile(max_rows, cols, groups, dtype == QA_BF16);
+  Tile tile = grouped_tile(max_rows, p.K, cols, groups, dtype == QA_BF16);
   if (gather && tile == TILE_L8R) tile = TILE_L8D2;  // gathered rows need the DMA ring
   const int bm = tile_rows(tile);
   p.tiles_m = (int)((max_rows + bm - 1) / bm + groups);
@@ -1094,7 +1130,7 @@ int qutai_amd_gemm_grouped_pair(const void* a, const void* a_tail, const void* b
   p.offsets = offsets;
   p.groups = groups;
   p.alpha = 1.0f;
-  Tile tile = grouped_tile(max_rows, cols, groups, dtype == QA_BF16);
+  Tile tile = grouped_tile(max_rows, p.K, cols, groups, dtype == QA_BF16);
   const int bm = tile_rows(tile);
   p.tiles_m = (int)((max_rows + bm - 1) / bm + groups);
   hipError_t err = dtype == QA_F32 ? launch_mma<true>(tile, false, transpose_right, p, stream)
@@ -1179,7 +1215,7 @@ int qutai_amd_gemm_grouped_k(const void* a, const void* b, void* out, const int6
   p.alpha = 1.0f;
   int64_t es = dtype == QA_BF16 ? 2 : 4;
   if ((p.lda * 256 * es) >= (1ll << 31) || (p.ldb * 256 * es) >= (1ll << 31)) return QA_EINVAL;
-  Tile tile = choose_tile(rows, cols, total_k / groups + 1, groups, dtype == QA_BF16);
+  Tile tile = choose_tile(rows, cols, total_k / groups + 1, groups, dtype == QA_BF16, true);
   if (gather) {
     // row offsets into b are 32-bit byte offsets of one buffer descriptor
     if (source_rows < 0 || source_rows * cols * es >= (1ll << 31)) return QA_EINVAL;

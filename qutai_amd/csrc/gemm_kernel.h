@@ -11,8 +11,9 @@
 //  * one workgroup computes a BM x BN output tile with WM x WN wavefronts;
 //    every wave owns a (BM/WM) x (BN/WN) sub-tile of 32x32 MFMA blocks whose
 //    fp32 accumulators stay in registers for the whole K loop;
-//  * bf16 operands feed v_mfma_f32_32x32x16_bf16, fp32 operands feed
-//    v_mfma_f32_32x32x2_f32 (true fp32 products, fp32 accumulation);
+//  * bf16 operands feed v_mfma_f32_32x32x16_bf16; fp32 operands feed it in
+//    three bf16 parts each, which hold all 24 bits (reduce_parts below), and
+//    v_mfma_f32_32x32x2_f32 where the parts do not serve;
 //  * A and B tiles move HBM -> LDS in 16-byte chunks with buffer loads,
 //    either straight into LDS (`buffer_load_dwordx4 ... lds`, DMA = true,
 //    STAGES-deep ring so several K steps are in flight while the MFMAs run;
@@ -30,6 +31,8 @@
 //  * workgroup ids are remapped so that each XCD (own L2) works on one
 //    compact block of output tiles.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace qa {
@@ -193,7 +196,11 @@ struct GemmKernel {
   // write rows 4 apart, into different bank halves.
   static constexpr int EP = TN + 8;
   static constexpr int RING_BYTES = STAGES * STAGE * (int)sizeof(T);
-  static constexpr int LDS_BYTES = RING_BYTES > NW * 32 * EP * 4 ? RING_BYTES : NW * 32 * EP * 4;
+  // fp32 in parts: two stages of 16 of K, three bf16 planes per operand
+  static constexpr int PLANE_A = BM * 16 + (KA ? 64 : 0), PLANE_B = BN * 16 + (KB ? 64 : 0);  // elements
+  static constexpr int PARTS = 3 * (PLANE_A + PLANE_B);
+  static constexpr int STAGES_BYTES = F32 && 2 * PARTS * 2 > RING_BYTES ? 2 * PARTS * 2 : RING_BYTES;
+  static constexpr int LDS_BYTES = STAGES_BYTES > NW * 32 * EP * 4 ? STAGES_BYTES : NW * 32 * EP * 4;
   static_assert(TileA::CHUNKS % NT == 0 && TileB::CHUNKS % NT == 0, "staging split");
   static_assert(TM % 32 == 0 && TN % 32 == 0 && BK % 16 == 0, "tile shape");
   static_assert(DMA || STAGES == 2, "register staging is double-buffered");
@@ -210,7 +217,7 @@ struct GemmKernel {
     uint32_t n = bytes > 0x7ffffff0 ? 0x7ffffff0u : (uint32_t)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, n, 0x00020000);
   }
-  __device__ static __forceinline__ u32x4 fetch(__amdgpu_buffer_rsrc_t r, uint32_t offset) {
+  __device__ static __forceinline__ u32x4 fetch16(__amdgpu_buffer_rsrc_t r, uint32_t offset) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0));
   }
 
@@ -231,15 +238,15 @@ struct GemmKernel {
   // 16-lane group, source lane i reads k-row kb + i/4, columns cb + 4 (i&3);
   // the hardware returns to lane i the 4 values of column cb + i.
   template <int R>
-  __device__ static __forceinline__ bf16x8 frag_mn16(const T* t, int col0, int s, int lane) {
+  __device__ static __forceinline__ bf16x8 frag_mn16(const bf16_t* t, int col0, int s, int lane) {
     constexpr int CR = R / 8;
     int g = lane >> 4, i = lane & 15;
     int cb = col0 + (g & 1) * 16 + 4 * (i & 3);
     int c = cb >> 3, w = cb & 7;
     int k0 = 16 * s + (g >> 1) * 8 + (i >> 2);
     int k1 = k0 + 4;
-    const T* p0 = t + k0 * R + ((c ^ swz_mn16<CR>(k0)) * 8) + w;
-    const T* p1 = t + k1 * R + ((c ^ swz_mn16<CR>(k1)) * 8) + w;
+    const bf16_t* p0 = t + k0 * R + ((c ^ swz_mn16<CR>(k0)) * 8) + w;
+    const bf16_t* p1 = t + k1 * R + ((c ^ swz_mn16<CR>(k1)) * 8) + w;
     typedef i16x4 __attribute__((address_space(3))) * lds_ptr;
     i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p0));
     i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p1));
@@ -338,6 +345,231 @@ struct GemmKernel {
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][q], fb[j][q], acc[i][j], 0, 0, 0);
       }
     }
+  }
+
+  // The tile this workgroup computes: operands from its first row / column and
+  // K on, and (when set) the tables that gather A's rows or B's K rows.
+  struct Work {
+    const T* a;
+    const T* b;
+    const T* a_tail;
+    const T* b_tail;
+    const int64_t* a_rows;
+    const int64_t* b_rows;
+    int64_t a_bytes, b_bytes, lda, ldb, M, N, K, k_head, row0, col0;
+  };
+
+  // fp32 operands on the bf16 matrix cores.  A value is the sum of three bf16
+  // parts v0 + v1 + v2 (split_bf16; every bit of it), and a product takes the
+  // six MFMAs whose terms are above 2^-24 of it, small ones first: 6 x 32
+  // cycles per 32x32x16 block where the fp32 MFMA takes 8 x 64.
+  //  * Each value is split once per workgroup, between the registers it was
+  //    loaded into and LDS: three planes per operand, 16 of K per stage, two
+  //    stages, so one barrier per stage and the next stage's split runs beside
+  //    the MFMAs.  (Split in every wave instead, on the way out of LDS, the
+  //    kernel is bound by that: 4096^3 796 against 666 us.)
+  //  * The bf16 MFMA cuts its sums off instead of rounding them, so a chain
+  //    drifts down by part of an ulp per step, which a column sum of the
+  //    results would show.  A chain therefore holds 16 of K only and is added
+  //    to the accumulator by a rounded add, and every other stage takes -A
+  //    and subtracts its sum.  K / 16 roundings per output against the fp32
+  //    MFMA's K / 2: error against float64 of normal values, K = 1000 and
+  //    3584, 1.5e-7 and 2.7e-7 against 5.7e-7 and 1.1e-6.
+  // Bound by the MFMAs at the power limit for whole rounds of 256x256 tiles
+  // (4096^3: 976 us with the fp32 MFMA, 666 now, 60% of the MFMA cycles); by
+  // the latency of a stage with one wave per SIMD on small tiles.
+  // An infinity or NaN has parts whose products give NaN, so it shows in the
+  // accumulators.  An element below 2^-110 loses up to 2^-134 (bf16's
+  // smallest step): with every output above 2^-80 that is below fp32's own
+  // rounding as long as the elements it meets are below 2^30 / K.  Returns
+  // whether this thread's outputs are all zero or finite and above 2^-80; a
+  // tile with one that is not is computed again with the fp32 MFMA.
+  __device__ static __forceinline__ bool reduce_parts(const Work& w, char* smem, f32x16 (&acc)[FM][FN], int tid) {
+    constexpr int NA = 2 * BM, ITEMS = (2 * (BM + BN) + NT - 1) / NT;  // eight-element items: A's, then B's
+    const int lane = tid & 63, wave = uniform32(tid >> 6), wm = wave / WN, wn = wave % WN;
+    bf16_t* planes = reinterpret_cast<bf16_t*>(smem);
+    // stages in flight in registers: a stage of a small tile is shorter than
+    // the loads take, a 256x256 tile has no registers for more
+    constexpr bool BIG = BM * BN >= 256 * 256;
+    constexpr int DEPTH = BIG ? 1 : 2;
+    u32x4 raw[DEPTH][ITEMS][2];
+    uint32_t off[ITEMS];
+    int at[ITEMS], kk[ITEMS];
+    bool in[ITEMS][2];
+    int64_t next_row[ITEMS];  // GATHER_B: source rows of the stage fetched next
+    static_assert(!GATHER_B || DEPTH == 1, "row indices are one stage ahead of one stage in flight");
+    const int64_t a_count = w.a_rows ? w.a_bytes / (w.lda * 4) : 0, b_count = GATHER_B ? w.b_bytes / (w.ldb * 4) : 0;
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+      const int idx = tid + j * NT;
+      const bool is_a = wave * 64 + j * NT < NA;  // wave-uniform
+      const bool kmajor = is_a ? KA : KB;
+      const int R = is_a ? BM : BN, q = is_a ? idx : idx - NA;
+      const int64_t ld = is_a ? w.lda : w.ldb;
+      // K-major: row q / 2, k = 8 (q % 2); MN-major: k row q / (R / 8), columns 8 (q % (R / 8))
+      const int outer = kmajor ? q >> 1 : q / (R / 8), c = kmajor ? q & 1 : q % (R / 8);
+      const int64_t first = kmajor ? outer : 8 * c, limit = is_a ? w.M - w.row0 : w.N - w.col0;
+      kk[j] = kmajor ? 8 * c : outer;
+      in[j][0] = idx < 2 * (BM + BN) && first < limit;
+      in[j][1] = idx < 2 * (BM + BN) && (kmajor ? first : first + 4) < limit;
+      int64_t row = outer;
+      if (is_a && KA && w.a_rows && in[j][0]) {
+        row = w.a_rows[w.row0 + outer];
+        if (row < 0 || row >= a_count) in[j][0] = in[j][1] = false;
+      }
+      off[j] = (uint32_t)(((GATHER_B && !is_a ? 0 : row * ld) + 8 * c) * 4);
+      if (kmajor) at[j] = c * (R * 8 + 64) + outer * 8;
+      else if (is_a) at[j] = outer * R + ((c ^ swz_mn16<BM / 8>(outer)) * 8);
+      else at[j] = outer * R + ((c ^ swz_mn16<BN / 8>(outer)) * 8);
+      if (!is_a) at[j] += 3 * PLANE_A;
+    }
+    auto fetch_rows = [&](int64_t k0) {  // GATHER_B: the source rows of the stage at k0
+      if constexpr (GATHER_B) {
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+          const bool is_a = wave * 64 + j * NT < NA;
+          next_row[j] = !is_a && in[j][0] && k0 + kk[j] < w.K ? w.b_rows[k0 + kk[j]] : -1;
+        }
+      }
+    };
+    auto fetch = [&](int slot, int64_t k0) {
+      const bool tail = w.k_head > 0 && k0 >= w.k_head;
+      const int64_t ks = tail ? k0 - w.k_head : k0;
+      const T* a = tail ? w.a_tail : w.a;
+      const T* b = tail ? w.b_tail : w.b;
+      // bases as in run()'s ring: A from its first row (gathered rows: the
+      // whole matrix), B from its first column
+      const auto da = w.a_rows ? rsrc(a + ks, w.a_bytes - ks * 4)
+                               : rsrc(KA ? a + w.row0 * w.lda + ks : a + ks * w.lda + w.row0,
+                                      (KA ? BM * w.lda : 16 * w.lda) * 4);
+      const auto db = GATHER_B ? rsrc(b + w.col0, w.b_bytes - w.col0 * 4)
+                               : rsrc(KB ? b + w.col0 * w.ldb + ks : b + ks * w.ldb + w.col0,
+                                      (KB ? BN * w.ldb : 16 * w.ldb) * 4);
+      const int64_t krem = w.K - k0;
+#pragma unroll
+      for (int j = 0; j < ITEMS; j++) {
+        const bool is_a = wave * 64 + j * NT < NA;
+        const bool kmajor = is_a ? KA : KB;
+        uint32_t o = off[j];
+        bool ok = true;
+        if constexpr (GATHER_B)
+          if (!is_a) {
+            ok = next_row[j] >= 0 && next_row[j] < b_count;
+            o += (uint32_t)(next_row[j] * w.ldb * 4);
+          }
+        raw[slot][j][0] = fetch16(is_a ? da : db, ok && in[j][0] && kk[j] < krem ? o : OOB);
+        raw[slot][j][1] = fetch16(is_a ? da : db, ok && in[j][1] && kk[j] + (kmajor ? 4 : 0) < krem ? o + 16 : OOB);
+      }
+    };
+    // the fetched stage into its planes; A times `sign`
+    auto put = [&](int slot, int stage, float sign) {
+#pragma unroll
+      for (int j = 0; j < ITEMS; j++) {
+        if (wave * 64 + j * NT >= 2 * (BM + BN)) continue;
+        const bool is_a = wave * 64 + j * NT < NA;
+        const float f = is_a ? sign : 1.f;
+        float v[8];
+        bf16x8 part[3];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = __uint_as_float(raw[slot][j][e >> 2][e & 3]) * f;
+        split_bf16(v, part);
+        bf16_t* to = planes + stage * PARTS + at[j];
+#pragma unroll
+        for (int n = 0; n < 3; n++) *reinterpret_cast<bf16x8*>(to + n * (is_a ? PLANE_A : PLANE_B)) = part[n];
+      }
+    };
+    // fragment of 32 rows from `row` on: lane = row, k = 8 (lane / 32) + [0, 8)
+    auto frag_a = [&](const bf16_t* t, int row) {
+      if constexpr (KA) return *reinterpret_cast<const bf16x8*>(t + (lane >> 5) * (BM * 8 + 64) + (row + (lane & 31)) * 8);
+      else return frag_mn16<BM>(t, row, 0, lane);
+    };
+    auto frag_b = [&](const bf16_t* t, int row) {
+      if constexpr (KB) return *reinterpret_cast<const bf16x8*>(t + (lane >> 5) * (BN * 8 + 64) + (row + (lane & 31)) * 8);
+      else return frag_mn16<BN>(t, row, 0, lane);
+    };
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) acc[i][j] = f32x16{};
+    const int nk = (int)((w.K + 15) / 16);
+    auto sync = [&] {  // LDS only: the loads in flight stay in flight
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      barrier();
+    };
+    // stage kt (kt % 2 == u): the next one from its registers into LDS, the
+    // one DEPTH after that into those registers, this one's products (stages
+    // past K are zeros).  Small tiles run it as one block of straight-line
+    // code, so that one wave per SIMD has the split beside its own MFMAs; the
+    // branches of a 256x256 tile keep it within 256 registers, and its two
+    // waves per SIMD run beside each other.
+    auto step = [&](int kt, auto u) {
+      constexpr int cur = decltype(u)::value, next = (cur + 1) % DEPTH;
+      constexpr float sign = cur ? -1.f : 1.f;
+      if (!BIG || kt + 1 < nk) {
+        put(next, cur ^ 1, -sign);
+        fetch(next, (int64_t)(kt + 1 + DEPTH) * 16);
+        fetch_rows((int64_t)(kt + 2 + DEPTH) * 16);
+      }
+      const bf16_t* sa = planes + cur * PARTS;
+      const bf16_t* sb = sa + 3 * PLANE_A;
+      bf16x8 pb[FN][3];
+#pragma unroll
+      for (int j = 0; j < FN; j++)
+#pragma unroll
+        for (int n = 0; n < 3; n++) pb[j][n] = frag_b(sb + n * PLANE_B, wn * TN + j * 32);
+#pragma unroll
+      for (int i = 0; i < FM; i++) {
+        bf16x8 pa[3];
+#pragma unroll
+        for (int n = 0; n < 3; n++) pa[n] = frag_a(sa + n * PLANE_A, wm * TM + i * 32);
+        f32x16 sum[FN] = {};
+#pragma unroll
+        for (int order = 2; order >= 0; order--)
+#pragma unroll
+          for (int x = 0; x <= order; x++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+              sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[x], pb[j][order - x], sum[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i][j] += sum[j] * sign;
+      }
+      if constexpr (!BIG) {
+        // per MFMA: one LDS read, a share of the split and the adds, one LDS write
+#pragma unroll
+        for (int m = 0; m < 6 * FM * FN; m++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+          __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        }
+      }
+      sync();  // this stage is read, the next one is written
+    };
+    fetch_rows(0);
+    fetch(0, 0);
+    fetch_rows(16);
+    put(0, 0, 1.f);
+#pragma unroll
+    for (int d = 1; d <= DEPTH; d++) {  // stage s sits in slot s % DEPTH
+      fetch(d % DEPTH, (int64_t)d * 16);
+      fetch_rows((int64_t)(d + 1) * 16);
+    }
+    sync();
+    for (int kt = 0; kt < nk; kt += 2) {
+      step(kt, std::integral_constant<int, 0>{});
+      if (!BIG || kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>{});
+    }
+    bool fine = true;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          const float x = __builtin_fabsf(acc[i][j][e]);
+          fine &= (x < INFINITY) & (x >= 0x1p-80f | x == 0.f);
+        }
+    return fine;
   }
 
   __device__ static __forceinline__ void run(const GemmArgs& p, char* smem) {
@@ -440,6 +672,20 @@ struct GemmKernel {
     const int64_t lda = p.lda, ldb = p.ldb;
 
     f32x16 acc[FM][FN];
+    bool redo = true;  // fp32: the parts did not serve this tile
+    if constexpr (F32) {
+      const Work w = {A, B, A_tail, B_tail, gather, gather_b, p.a_bytes, p.b_bytes, lda, ldb, M, N, K, k_head, row0,
+                      col0};
+      const bool fine = reduce_parts(w, smem, acc, tid);
+      int* flag = reinterpret_cast<int*>(smem);  // the planes are no longer read
+      if (tid == 0) *flag = 0;
+      __syncthreads();
+      if (__builtin_amdgcn_ballot_w64(!fine) && lane == 0) *flag = 1;
+      __syncthreads();
+      redo = uniform32(*flag) != 0;
+      __syncthreads();  // the flag is read before the ring is filled
+    }
+    if (redo) {
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
@@ -638,9 +884,9 @@ struct GemmKernel {
         auto db = desc_b(k0);
         const int64_t krem = K - k0;
 #pragma unroll
-        for (int i = 0; i < LA; i++) ra[i] = fetch(da, (va[i] && ka[i] < krem) ? oa[i] : OOB);
+        for (int i = 0; i < LA; i++) ra[i] = fetch16(da, (va[i] && ka[i] < krem) ? oa[i] : OOB);
 #pragma unroll
-        for (int i = 0; i < LB; i++) rb[i] = fetch(db, (vb[i] && kb[i] < krem) ? ob[i] : OOB);
+        for (int i = 0; i < LB; i++) rb[i] = fetch16(db, (vb[i] && kb[i] < krem) ? ob[i] : OOB);
       };
       auto store = [&](int stage) {
         T* sa = lds + stage * STAGE;
@@ -673,6 +919,8 @@ struct GemmKernel {
         if (kt + 1 < nk) store(cur ^ 1);
         __syncthreads();
       }
+    }
+
     }
 
     // ---- epilogue ---------------------------------------------------------

@@ -1,0 +1,61 @@
+"""fp32 GEMMs run on the bf16 matrix cores with every operand in three bf16
+parts: against float64 at the edges of the tiles, and for operands that the
+parts do not serve (infinities, NaN, values next to the ends of the range),
+which must come out as the fp32 MFMA has them.
+
+Tolerance: a K-long sum rounds at most 6 times per 16 of K, each time by 2^-24
+of the running sum at most; with K <= 4096 normal products the measured error
+is below 1e-6, the bar 2e-6."""
+import numpy as np
+import pytest
+
+from oracle import reference as ora
+from tests.helpers import download, normal, upload
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd():
+    from qutai_amd.backends import amd
+
+    amd.get_runtime()
+    return amd
+
+
+def product(amd, a, b, ta=False, tb=False, **kw):
+    m, k, n = a.shape[0], a.shape[1], b.shape[1]
+    left, right = upload((a.T if ta else a).ravel(), "float32"), upload((b.T if tb else b).ravel(), "float32")
+    return download(amd.gemm(left, right, m, k, n, transpose_left=ta, transpose_right=tb, **kw)).reshape(m, n)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 16, 1), (33, 17, 65), (128, 256, 64), (257, 130, 255), (64, 4096, 64),
+                                   (520, 1000, 700), (1100, 96, 1030)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("scale", [1.0, 1e-30])
+def test_against_float64(amd, m, k, n, ta, tb, scale):
+    a, b = normal(m, (m, k), scale), normal(n, (k, n))
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    assert ora.rel_frobenius(product(amd, a, b, ta, tb), exact) <= 2e-6
+
+
+def test_subnormal_operands_keep_their_bits(amd):
+    a, b = normal(1, (96, 200), 3e-39), normal(2, (200, 160), 1e5)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    assert ora.rel_frobenius(product(amd, a, b), exact) <= 2e-6
+
+
+def test_infinities_nan_and_the_top_of_the_range(amd):
+    a, b = normal(3, (300, 64)), normal(4, (64, 300))
+    a[5, 7], a[9, 3], b[11, 13] = np.inf, np.nan, -np.inf
+    a[20] = 0
+    a[20, 0], b[0, 40] = 3.4e38, 0.5  # finite: next to the largest float, halved
+    with np.errstate(invalid="ignore"):
+        exact = a.astype(np.float64) @ b.astype(np.float64)
+    got = product(amd, a, b)
+    assert np.array_equal(np.isnan(got), np.isnan(exact))
+    top = float(np.finfo(np.float32).max) * (1 + 2.0 ** -25)  # beyond it fp32 rounds to infinity
+    assert np.array_equal(np.isposinf(got), exact > top) and np.array_equal(np.isneginf(got), exact < -top)
+    finite = np.isfinite(got)
+    assert ora.rel_frobenius(got[finite], exact[finite]) <= 2e-6
+    assert abs(got[20, 40] / exact[20, 40] - 1) <= 2e-6
