@@ -249,36 +249,99 @@ __global__ void __launch_bounds__(THREADS) row_partials_kernel(const typename Ac
   }
 }
 
-// inner > 1: one lane per (o, part, j) column segment, consecutive lanes on
-// consecutive j (coalesced); parts == 1 writes the rounded sum.
-template <class T>
+// inner > 1: a workgroup sums `span` rows of 64 V neighbouring columns (V
+// elements, 16 bytes, per lane where rows allow it, else one); its four waves
+// take every fourth row with eight rows' loads in flight, and their sums are
+// added in wave order.  parts == 1 writes the rounded sum, otherwise the fp
+// partials [o][part][j] go to `partial`.  Bound by HBM: 2048 x 3584 fp32 with
+// col_partials 40 -> 12 us, 4096 x 512 fp32 34 -> 9 (one row's load at a
+// time per lane, and the partials added by one lane per column, before).
+template <class T, int V>
 __global__ void __launch_bounds__(THREADS) col_sum_kernel(const T* __restrict__ x, T* __restrict__ out,
                                                           typename Acc<T>::R* __restrict__ partial, int64_t outer,
                                                           int64_t width, int64_t inner, int64_t parts, int64_t span) {
   typedef typename Acc<T>::R R;
-  const int64_t total = outer * parts * inner;
-  for (int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x; i < total; i += (int64_t)gridDim.x * THREADS) {
-    const int64_t j = i % inner, op = i / inner, part = op % parts, o = op / parts;
+  constexpr int W = THREADS / 64, DEEP = 8;
+  __shared__ R sums[W - 1][64 * V];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t blocks = (inner + 64 * V - 1) / (64 * V), total = outer * parts * blocks;
+  for (int64_t item = blockIdx.x; item < total; item += gridDim.x) {
+    const int64_t j = (item % blocks * 64 + lane) * V, op = item / blocks, part = op % parts, o = op / parts;
     const int64_t lo = part * span, hi = lo + span < width ? lo + span : width;
+    const bool in = j < inner;
+    R s[V];
+#pragma unroll
+    for (int t = 0; t < V; t++) s[t] = R(0);
     const T* p = x + o * width * inner + j;
-    R s = R(0);
-    for (int64_t c = lo; c < hi; c++) s += widen(p[c * inner]);
-    if (parts == 1) out[o * inner + j] = narrow<T>(s);
-    else partial[i] = s;
+    for (int64_t c = lo + wave; c < hi; c += W * DEEP) {
+      T v[DEEP][V];
+#pragma unroll
+      for (int u = 0; u < DEEP; u++) {
+        const bool row = in && c + u * W < hi;
+        if constexpr (V > 1) {
+          u32x4 w = {0u, 0u, 0u, 0u};
+          if (row) w = global_load<u32x4>(p + (c + u * W) * inner);
+          *reinterpret_cast<u32x4*>(v[u]) = w;
+        } else {
+          v[u][0] = row ? p[(c + u * W) * inner] : T(0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < DEEP; u++)
+#pragma unroll
+        for (int t = 0; t < V; t++)
+          if (in && c + u * W < hi) s[t] += widen(v[u][t]);
+    }
+    if (wave) {
+#pragma unroll
+      for (int t = 0; t < V; t++) sums[wave - 1][lane * V + t] = s[t];
+    }
+    __syncthreads();
+    if (!wave && in) {
+#pragma unroll
+      for (int t = 0; t < V; t++) {
+#pragma unroll
+        for (int w = 0; w < W - 1; w++) s[t] += sums[w][lane * V + t];
+        if (parts == 1) out[o * inner + j + t] = narrow<T>(s[t]);
+        else partial[op * inner + j + t] = s[t];
+      }
+    }
+    __syncthreads();  // the sums are read before the next item's are written
   }
 }
 
+// The partials of each column: four waves take every fourth part of 64
+// columns, eight loads in flight, their sums added in wave order.
 template <class T>
 __global__ void __launch_bounds__(THREADS) col_partials_kernel(const typename Acc<T>::R* __restrict__ partial,
                                                                T* __restrict__ out, int64_t outer, int64_t inner,
                                                                int64_t parts) {
   typedef typename Acc<T>::R R;
-  const int64_t total = outer * inner;
-  for (int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x; i < total; i += (int64_t)gridDim.x * THREADS) {
-    const int64_t o = i / inner, j = i % inner;
+  constexpr int W = THREADS / 64, DEEP = 8;
+  __shared__ R sums[W - 1][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t blocks = (inner + 63) / 64, total = outer * blocks;
+  for (int64_t item = blockIdx.x; item < total; item += gridDim.x) {
+    const int64_t j = item % blocks * 64 + lane, o = item / blocks;
+    const R* p = partial + o * parts * inner + j;
     R s = R(0);
-    for (int64_t q = 0; q < parts; q++) s += partial[(o * parts + q) * inner + j];
-    out[i] = narrow<T>(s);
+    if (j < inner)
+      for (int64_t q = wave; q < parts; q += W * DEEP) {
+        R v[DEEP];
+#pragma unroll
+        for (int u = 0; u < DEEP; u++) v[u] = q + u * W < parts ? p[(q + u * W) * inner] : R(0);
+#pragma unroll
+        for (int u = 0; u < DEEP; u++)
+          if (q + u * W < parts) s += v[u];
+      }
+    if (wave) sums[wave - 1][lane] = s;
+    __syncthreads();
+    if (!wave && j < inner) {
+#pragma unroll
+      for (int w = 0; w < W - 1; w++) s += sums[w][lane];
+      out[o * inner + j] = narrow<T>(s);
+    }
+    __syncthreads();
   }
 }
 
@@ -327,7 +390,7 @@ int by_float_dtype(int dtype, F f) {
 }
 
 // Parts a reduction of `count` independent sums of `width` terms is split
-// into, so that at least ~2048 waves (or lanes for the column form) run.
+// into, so that at least ~2048 waves run.
 int64_t reduce_parts(int64_t count, int64_t width, int64_t target, int64_t min_span) {
   if (count >= target || width < 2 * min_span) return 1;
   int64_t parts = (target + count - 1) / count;
@@ -341,8 +404,10 @@ void row_plan(int64_t rows, int64_t width, int64_t& parts, int64_t& span) {
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;
 }
+// Column form: about 1024 workgroups (each of 256 columns, the narrowest 16-byte
+// lanes) of at least 32 rows, one round of loads.
 void col_plan(int64_t columns, int64_t width, int64_t& parts, int64_t& span) {
-  parts = reduce_parts(columns, width, 65536, 64);
+  parts = reduce_parts((columns + 255) / 256, width, 1024, 32);
   span = (width + parts - 1) / parts;
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;
@@ -477,10 +542,16 @@ int qutai_amd_reduce_sum(const void* x, void* out, int64_t outer, int64_t width,
         row_partials_kernel<T><<<blocks_for(outer, THREADS / 64), THREADS, 0, st>>>(partial, (T*)out, outer, parts);
     } else {
       col_plan(outer * inner, width, parts, span);
-      col_sum_kernel<T><<<blocks_for(outer * parts * inner), THREADS, 0, st>>>((const T*)x, (T*)out, partial, outer,
-                                                                               width, inner, parts, span);
+      constexpr int V = Lanes<T>::V;
+      if (inner % V == 0 && (uintptr_t)x % 16 == 0)
+        col_sum_kernel<T, V><<<blocks_for(outer * parts * ((inner + 64 * V - 1) / (64 * V)), 1), THREADS, 0, st>>>(
+            (const T*)x, (T*)out, partial, outer, width, inner, parts, span);
+      else
+        col_sum_kernel<T, 1><<<blocks_for(outer * parts * ((inner + 63) / 64), 1), THREADS, 0, st>>>(
+            (const T*)x, (T*)out, partial, outer, width, inner, parts, span);
       if (parts > 1)
-        col_partials_kernel<T><<<blocks_for(outer * inner), THREADS, 0, st>>>(partial, (T*)out, outer, inner, parts);
+        col_partials_kernel<T><<<blocks_for(outer * ((inner + 63) / 64), 1), THREADS, 0, st>>>(partial, (T*)out, outer,
+                                                                                             inner, parts);
     }
     return (int)hipGetLastError();
   });

@@ -177,6 +177,35 @@ __global__ void splitk_reduce(const float* part, void* out, int64_t n, int64_t t
   }
 }
 
+// The same for columns, row pitch, product size and output start that are
+// multiples of four elements: 16 bytes of each partial per thread, 32-bit
+// indices (total / 4 below 2^32).  3584 x 1024 outputs in 2 chunks: 15 -> 8 us.
+__global__ void __launch_bounds__(256) splitk_reduce4(const float* part, void* out, uint32_t n4, uint32_t total4,
+                                                      int splits, int accumulate, int out_bf16, uint32_t cols4,
+                                                      int64_t ldc) {
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total4; i += gridDim.x * 256) {
+    const uint32_t b = i / n4, e = i - b * n4;
+    const float* src = part + ((int64_t)b * splits * n4 + e) * 4;
+    f32x4 acc = {};
+    for (int s = 0; s < splits; s++) acc += global_load<f32x4>(src + (int64_t)s * n4 * 4);
+    const uint32_t row = e / cols4;
+    const int64_t at = ((int64_t)b * (n4 / cols4) + row) * ldc + (int64_t)(e - row * cols4) * 4;
+    if (out_bf16) {
+      bf16_t* q = (bf16_t*)out + at;
+      if (accumulate) {
+        const u32x2 old = global_load<u32x2>(q);
+        acc += f32x4{__uint_as_float(old[0] << 16), __uint_as_float(old[0] & 0xffff0000u),
+                     __uint_as_float(old[1] << 16), __uint_as_float(old[1] & 0xffff0000u)};
+      }
+      global_store(q, u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])});
+    } else {
+      float* q = (float*)out + at;
+      if (accumulate) acc += global_load<f32x4>(q);
+      global_store(q, acc);
+    }
+  }
+}
+
 // Column remainder of at most 8 columns with a K-major A (the last r
 // columns of a 256 q + r wide product): a workgroup of RWAVES waves computes
 // RWAVES * RROWS output rows.  It stages B's r columns for KC values of k at
@@ -1031,6 +1060,15 @@ int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_
     if (err != hipSuccess) return (int)err;
     if (!window_part) continue;
     const int64_t total = batch * rows * x.n;
+    if (x.n % 4 == 0 && cols % 4 == 0 && (uintptr_t)window_out % (4 * osize) == 0 && total / 4 < (1ll << 31)) {
+      const unsigned blocks4 = (unsigned)((total / 4 + 255) / 256);
+      hipLaunchKernelGGL(splitk_reduce4, dim3(blocks4), dim3(256), 0, stream, (const float*)window_part,
+                         (void*)window_out, (uint32_t)(rows * x.n / 4), (uint32_t)(total / 4), x.splits,
+                         accumulate ? 1 : 0, out_dtype == QA_BF16 ? 1 : 0, (uint32_t)(x.n / 4), cols);
+      err = hipGetLastError();
+      if (err != hipSuccess) return (int)err;
+      continue;
+    }
     const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 20);
     hipLaunchKernelGGL(splitk_reduce, dim3(blocks), dim3(256), 0, stream, (const float*)window_part,
                        (void*)window_out, rows * x.n, total, x.splits, accumulate ? 1 : 0,

@@ -494,6 +494,25 @@ __global__ void silu_mul_kernel(const void* g, const void* u, void* out, int64_t
   }
 }
 
+// The same where rows are whole 16-byte chunks: 4 fp32 or 8 bf16 values per
+// thread and step, 32-bit chunk indices (n below 2^32).  Bound by HBM: 2048 x
+// 3584 fp32 21 -> 12 us (one value per thread and a 64-bit remainder before).
+template <bool F32>
+__global__ void __launch_bounds__(THREADS) add_rows_vec(const u32x4* x, const u32x4* bias, u32x4* out, uint32_t n,
+                                                        uint32_t per_row) {
+  for (uint32_t i = blockIdx.x * THREADS + threadIdx.x; i < n; i += gridDim.x * THREADS) {
+    const u32x4 a = global_load<u32x4>(x + i), b = global_load<u32x4>(bias + i % per_row);
+    u32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      if constexpr (F32) y[e] = __float_as_uint(__uint_as_float(a[e]) + __uint_as_float(b[e]));
+      else y[e] = pack_bf16x2(__uint_as_float(a[e] << 16) + __uint_as_float(b[e] << 16),
+                              __uint_as_float(a[e] & 0xffff0000u) + __uint_as_float(b[e] & 0xffff0000u));
+    }
+    global_store(out + i, y);
+  }
+}
+
 __global__ void add_rows_kernel(const void* x, const void* bias, void* out, int64_t rows, int64_t cols, int d) {
   int64_t n = rows * cols;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -692,6 +711,19 @@ int qutai_amd_add_rows(const void* x, const void* bias, void* out, int64_t rows,
                        void* stream) {
   if (rows < 0 || cols < 0 || !float_dtype(dtype)) return QA_EINVAL;
   if (rows * cols == 0) return QA_OK;
+  const int64_t per_chunk = dtype == F32 ? 4 : 8, chunks = rows * cols / per_chunk;
+  if (dtype != F64 && cols % per_chunk == 0 && chunks < (1ll << 31) &&
+      ((uintptr_t)x | (uintptr_t)bias | (uintptr_t)out) % 16 == 0) {
+    const dim3 grid(grid_for(chunks));
+    const uint32_t n = (uint32_t)chunks, per_row = (uint32_t)(cols / per_chunk);
+    if (dtype == F32)
+      hipLaunchKernelGGL(add_rows_vec<true>, grid, dim3(THREADS), 0, (hipStream_t)stream, (const u32x4*)x,
+                         (const u32x4*)bias, (u32x4*)out, n, per_row);
+    else
+      hipLaunchKernelGGL(add_rows_vec<false>, grid, dim3(THREADS), 0, (hipStream_t)stream, (const u32x4*)x,
+                         (const u32x4*)bias, (u32x4*)out, n, per_row);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(add_rows_kernel, dim3(grid_for(rows * cols)), dim3(THREADS), 0, (hipStream_t)stream, x, bias,
                      out, rows, cols, dtype);
   return (int)hipGetLastError();
