@@ -404,10 +404,10 @@ void row_plan(int64_t rows, int64_t width, int64_t& parts, int64_t& span) {
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;
 }
-// Column form: about 1024 workgroups (each of 256 columns, the narrowest 16-byte
-// lanes) of at least 32 rows, one round of loads.
+// Column form: about 65536 column segments of at least 64 rows, 256 to a
+// workgroup of the fp32 kernel.
 void col_plan(int64_t columns, int64_t width, int64_t& parts, int64_t& span) {
-  parts = reduce_parts((columns + 255) / 256, width, 1024, 32);
+  parts = reduce_parts(columns, width, 65536, 64);
   span = (width + parts - 1) / parts;
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;

@@ -662,15 +662,17 @@ Tile grouped_tile(int64_t rows, int64_t inner, int64_t cols, int groups, bool bf
 // K chunks of a plain product (batch 1): the tile and the chunk count with the
 // lowest launch_cost over one chunk plus the partial sums' traffic ((2 s + 1)
 // x rows x cols fp32 values at 5 TB/s) and 4 us for the launch that adds them
-// up, if that is at least 15% below the product in one piece; below K = 512
-// the second launch and its workspace cost the host more than the GPU gains.  Which products try:
-//  * fp32 and thin outputs (<= 64 columns or rows): every one; their tiles are
-//    long (fp32) or few (512 x 4096 x 512 fp32, K 4096: 128 us in one piece,
-//    32 in eight; a router's 8 logits; 30 x 2048 x 300 bf16: 17 -> 14 us);
+// up, if that is at least 15% below the product in one piece (the last kind
+// below: up to 5% above, where it measured 24 us against 28); below K = 512 the
+// second launch and its workspace cost the host more than the GPU gains.  Which products try:
+//  * fp32 and thin outputs (<= 64 columns or rows): every one, on the small
+//    tiles; their tiles are long (fp32) or few (512 x 4096 x 512 fp32: 128 us
+//    in one piece, 32 in eight; a router's 8 logits; 30 x 2048 x 300 bf16:
+//    17 -> 14 us);
 //  * other bf16 products: K >= 4096 over at most a quarter of the 128x128
 //    tile slots (the decoder head's dX, 1024 x 2048 outputs over K = 32768:
-//    158 -> 129 us with 256x256 tiles in 8 chunks); with shorter K the chunks
-//    measured slower.
+//    158 -> 129 us with 256x256 tiles in 8 chunks), on the large tiles; with
+//    shorter K the chunks measured slower.
 int choose_split(int64_t rows, int64_t cols, int64_t inner, int64_t batch, Tile* tile, bool bf16, bool ta,
                  int64_t* chunk) {
   const int64_t cus = cu_count();
@@ -682,9 +684,10 @@ int choose_split(int64_t rows, int64_t cols, int64_t inner, int64_t batch, Tile*
   } else if (batch == 1 && forced_tile() < 0 && inner >= 512 && *tile != TILE_N && *tile != TILE_W &&
              (!bf16 || thin || (inner >= 4096 && tile_count(TILE_S, rows, cols, 1) * 2 <= cus))) {
     const double whole = launch_cost(*tile, tile_count(*tile, rows, cols, 1), inner, bf16, ta);
-    double best = 0.85 * whole;
-    for (Tile t : {TILE_L8D2, TILE_H, TILE_X, TILE_S, TILE_Z}) {
-      if ((thin && t != TILE_Z) || (!bf16 && (t == TILE_H || t == TILE_S))) continue;
+    double best = (bf16 && !thin ? 1.05 : 0.85) * whole;
+    for (Tile t : {TILE_L8D2, TILE_H, TILE_S, TILE_X, TILE_Z}) {
+      const bool small = t == TILE_X || t == TILE_Z;
+      if (thin ? t != TILE_Z : small == bf16) continue;
       const int64_t n = tile_count(t, rows, cols, 1);
       for (int64_t st = 2; st <= (thin ? 16 : 8) && inner >= 64 * st; st++) {
         const int64_t c = ((inner + st - 1) / st + 63) / 64 * 64;
