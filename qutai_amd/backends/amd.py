@@ -46,8 +46,8 @@ class AMDStorage(Storage):
         if size < 0:
             raise ValueError("storage size must be non-negative")
         self.dtype, self._size = dtype, size
-        self.runtime = get_runtime()
-        self.ptr = self.runtime.allocate(self.nbytes)
+        self.runtime = runtime = get_runtime()
+        self.ptr = runtime.allocate(size * _TYPES[dtype][1])
 
     @property
     def size(self) -> int:
@@ -246,11 +246,12 @@ def gemm(left, right, rows, inner, cols, *, batch=1, transpose_left=False, trans
     dtype = ("float64" if double else "float32") if out_dtype is None else out_dtype
     if dtype not in (("float64",) if double else ("float32", "bfloat16")):
         raise ValueError("GEMM output dtype is incompatible with the inputs")
-    if any(type(x) is not int or x < 0 for x in (rows, inner, cols, batch)):
+    if (type(rows) is not int or type(inner) is not int or type(cols) is not int or type(batch) is not int
+            or rows < 0 or inner < 0 or cols < 0 or batch < 0):
         raise ValueError("GEMM dimensions must be non-negative integers")
     sa = rows * inner if left_stride is None else left_stride
     sb = inner * cols if right_stride is None else right_stride
-    if any(type(x) is not int or x < 0 for x in (sa, sb)):
+    if type(sa) is not int or type(sb) is not int or sa < 0 or sb < 0:
         raise ValueError("GEMM batch strides must be non-negative integers")
     if batch and (left.size < (batch - 1) * sa + rows * inner or right.size < (batch - 1) * sb + inner * cols):
         raise ValueError("GEMM input storage is too small")
@@ -268,17 +269,13 @@ def gemm(left, right, rows, inner, cols, *, batch=1, transpose_left=False, trans
         return result
     mixed = not double and (left.dtype == "bfloat16" or right.dtype == "bfloat16" or matmul_precision() == "bfloat16")
     runtime = get_runtime()
-    workspace = None
-    if not double:
-        need = runtime.lib.qutai_amd_gemm_workspace_size(rows, inner, cols, batch, sa, sb, int(bool(transpose_left)),
-                                                         int(bool(transpose_right)), code(left.dtype),
-                                                         code(right.dtype), int(mixed))
-        if need:
-            workspace = AMDStorage((need + 1) // 2, "bfloat16")
-    runtime.call("qutai_amd_gemm", left.ptr, right.ptr, result.ptr, rows, inner, cols, batch, sa, sb,
-                 int(bool(transpose_left)), int(bool(transpose_right)), code(left.dtype), code(right.dtype),
-                 code(dtype), int(bool(accumulate)), int(mixed), _p(workspace),
-                 workspace.nbytes if workspace is not None else 0, mfma=not double)
+    ta, tb, mixed = int(bool(transpose_left)), int(bool(transpose_right)), int(mixed)
+    left_code, right_code = _CODES[left.dtype], _CODES[right.dtype]
+    need = 0 if double else runtime.gemm_workspace(rows, inner, cols, batch, sa, sb, ta, tb, left_code, right_code, mixed)
+    workspace = AMDStorage((need + 1) // 2, "bfloat16") if need else None
+    runtime.call("qutai_amd_gemm", left.ptr, right.ptr, result.ptr, rows, inner, cols, batch, sa, sb, ta, tb, left_code,
+                 right_code, _CODES[dtype], int(bool(accumulate)), mixed, workspace.ptr if need else 0,
+                 workspace.nbytes if need else 0, mfma=not double)
     return result
 
 

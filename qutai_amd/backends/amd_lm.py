@@ -12,8 +12,8 @@ memory, so no host synchronisation sizes them).
 from __future__ import annotations
 
 from array import array
-from bisect import bisect_left
-from functools import partial
+from itertools import compress, islice
+from operator import ne
 from random import Random
 
 from . import amd
@@ -534,11 +534,12 @@ def embedding_backward_index(ids):
         ids = array("q", (int(t) for t in ids))
     order = sorted(range(len(ids)), key=ids.__getitem__)  # stable: input order within a token
     grouped = array("q", map(ids.__getitem__, order))
-    tokens = sorted(set(ids))
-    offsets = array("q", map(partial(bisect_left, grouped), tokens))
+    # a token's rows start where the grouped ids change
+    offsets = array("q", range(min(1, len(ids))))
+    offsets.extend(compress(range(1, len(ids)), map(ne, islice(grouped, 1, None), grouped)))
+    tokens = array("q", map(grouped.__getitem__, offsets))
     offsets.append(len(ids))
-    return tuple(amd.storage(values, dtype="int64")
-                 for values in (array("q", tokens), offsets, array("q", order)))
+    return tuple(amd.storage(values, dtype="int64") for values in (tokens, offsets, array("q", order)))
 
 
 def embedding_backward(gradient, ids, count, width, *, index=None, out=None):

@@ -148,6 +148,8 @@ class Runtime:
         self.hip = _hip_library()
         self._bind_hip()
         self.lib = load_library()
+        self._functions = {name: getattr(self.lib, name) for name in SIGNATURES}
+        self._gemm_workspaces = {}  # shape and types of a product -> workspace bytes
         self._check(self._init(0), "hipInit")
         count = ctypes.c_int()
         self._check(self._device_count(ctypes.byref(count)), "hipGetDeviceCount")
@@ -359,21 +361,38 @@ class Runtime:
     def call(self, name: str, *arguments, mfma: bool = False):
         """Run one libqutai_amd entry point on the default stream."""
         with self._lock:
-            self._current()
-            status = getattr(self.lib, name)(*arguments, None)
-            if status == QA_EINVAL:
-                raise ValueError(f"{name}: arguments rejected by libqutai_amd")
-            if status == QA_EWORKSPACE:
-                raise RuntimeError(f"{name}: workspace missing or too small")
-            if status == QA_ESCRATCH:
-                raise RuntimeError(f"{name}: the operands need more workspace than the fixed "
-                                   f"{self.lib.qutai_amd_gemm_static_capacity() >> 20} MiB device scratch")
-            self._check(status, name)
+            if self._closed:
+                self._current()
+            status = self._functions[name](*arguments, None)
+            if status:
+                self._fail(status, name)
             self.launches += 1
             if mfma:
                 self.mfma_launches += 1
             if self.debug_sync:
                 self._check(self._sync(), f"hipDeviceSynchronize after {name}")
+
+    def _fail(self, status, name):
+        if status == QA_EINVAL:
+            raise ValueError(f"{name}: arguments rejected by libqutai_amd")
+        if status == QA_EWORKSPACE:
+            raise RuntimeError(f"{name}: workspace missing or too small")
+        if status == QA_ESCRATCH:
+            raise RuntimeError(f"{name}: the operands need more workspace than the fixed "
+                               f"{self.lib.qutai_amd_gemm_static_capacity() >> 20} MiB device scratch")
+        self._check(status, name)
+
+    def gemm_workspace(self, *shape):
+        """qutai_amd_gemm_workspace_size of a product's shape and types, asked
+        once per shape (and forced split): the plan depends on nothing else,
+        and the call costs a small product as much host time as its launch."""
+        key = (*shape, os.environ.get("QUTAI_AMD_SPLITK"))
+        need = self._gemm_workspaces.get(key)
+        if need is None:
+            if len(self._gemm_workspaces) >= 4096:
+                self._gemm_workspaces.clear()
+            need = self._gemm_workspaces[key] = self.lib.qutai_amd_gemm_workspace_size(*shape)
+        return need
 
     # ---- events (timing on the default stream) ---------------------------------
     def event(self):
@@ -416,6 +435,9 @@ class Runtime:
 def get_runtime() -> Runtime:
     """First device touch loads the libraries and binds device 0."""
     global _runtime
+    runtime = _runtime
+    if runtime is not None and not runtime._closed:
+        return runtime
     with _runtime_lock:
         if _runtime is None or _runtime._closed:
             _runtime = Runtime()

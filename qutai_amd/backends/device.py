@@ -16,8 +16,9 @@ _BACKENDS = {"amd": amd}
 def get_backend(device="amd", *others):
     """Backend for a device string or storage; several storages must share device and dtype."""
     if isinstance(device, Storage):
-        if any((item.device, item.dtype) != (device.device, device.dtype) for item in others):
-            raise ValueError("operands must share device and dtype")
+        for item in others:
+            if item.dtype != device.dtype or item.device != device.device:
+                raise ValueError("operands must share device and dtype")
         device = device.device
     if device not in _BACKENDS:
         raise ValueError(f"unsupported device: {device}")

@@ -24,6 +24,12 @@ def owned(storage):
     return storage
 
 
+def owned_by_leaf(storage, parent):
+    """``owned`` for a gradient that goes straight to a leaf.  (One that flows
+    on through other rules may be passed to several tensors by them.)"""
+    return owned(storage) if getattr(parent, "backward_rule", None) is None else storage
+
+
 def take_owned(storage):
     """True (once) when ``storage`` was marked by ``owned``."""
     if getattr(storage, "owned_gradient", False):

@@ -34,7 +34,7 @@ class Tensor:
         else:
             self.shape = infer_shape(data) if shape is None else tuple(shape)
             self.storage = backend.storage(flatten(data), dtype=dtype)
-        if any(size < 0 for size in self.shape) or prod(self.shape) != self.storage.size:
+        if prod(self.shape) != self.storage.size or (self.shape and min(self.shape) < 0):
             raise ValueError("element count does not match the Tensor shape")
         self.requires_grad = requires_grad
         self.grad = None
