@@ -396,6 +396,16 @@ int qutai_amd_attention_fwd(const void* q, const void* k, const void* v, void* o
                             int64_t heads, int64_t kv_heads, int64_t time, int64_t dim, int dtype, int layout,
                             double scale, int causal, void* stream);
 
+/* Attention of `length` new positions over a key/value cache of `total`
+ * positions whose last `length` are the new ones: query i sees the first
+ * total - length + i + 1 keys.  q and out are [batch][length][heads][dim], k
+ * and v [batch][heads][total][dim], all of `dtype` (QA_BF16 with dim % 8 == 0,
+ * QA_F32 with dim % 4 == 0; dim <= 256) and 16-byte aligned; total <= 12000.
+ * Scores, probabilities and sums are fp32.  Replaces the Q K^T / softmax / P V
+ * sequence of the cache path (src/qutai/nn/layers.py:345-355). */
+int qutai_amd_attention_cached(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t heads,
+                               int64_t length, int64_t total, int64_t dim, int dtype, double scale, void* stream);
+
 /* Grouped-K GEMM for the MoE weight gradients: for every group g,
  *   out[g] (rows x cols) (+)= A_g^T B_g,
  * where A_g / B_g are the K rows [offsets[g], offsets[g+1]) of a ([K][rows])

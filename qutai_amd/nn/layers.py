@@ -14,8 +14,9 @@ dim) is the lm layout), so the length x length scores are never stored;
 reference.  ``MultiHeadAttention(..., cache=KVCache())`` runs causal
 inference over new positions only: their projections, the cached keys and
 values appended, the score product against every cached key with the
-causal mask shifted by the cached length, softmax and the value product, all
-with graph recording off (src/qutai/nn/layers.py:334-355).
+causal mask shifted by the cached length, softmax and the value product (a
+few positions in one launch), all with graph recording off
+(src/qutai/nn/layers.py:334-355).
 """
 from __future__ import annotations
 
@@ -23,6 +24,7 @@ from math import sqrt
 from random import Random
 
 from ..backends import amd, amd_lm
+from ..backends.precision import matmul_precision
 from ..core import operations
 from ..core.context import set_recording
 from ..core.grad import owned_by_leaf, record
@@ -108,6 +110,8 @@ class Attention:
     def _split(self, tensor):
         """(batch, length, features) -> (batch, heads, length, features / heads)."""
         batch, length, features = tensor.shape
+        if length == 1:  # the same order of elements
+            return tensor.reshape((batch, self.heads, 1, features // self.heads))
         return tensor.reshape((batch, length, self.heads, features // self.heads)).transpose((0, 2, 1, 3))
 
     def _probabilities(self, queries, keys):
@@ -166,14 +170,17 @@ class MultiHeadAttention(Attention):
             return self.output(self._mix(*(layer(tensor) for layer in (self.query, self.key, self.value))))
         with set_recording(False):
             tensor = self._input(data)
-            queries, keys, values = (self._split(layer(tensor)) for layer in (self.query, self.key, self.value))
-            keys, values = cache.update(keys, values)
-            length, total = queries.shape[2], keys.shape[2]
-            scores = matmul(queries, keys.transpose((0, 1, 3, 2)))
-            probabilities = softmax(causal_mask(scores, offset=total - length), -1,
-                                    scale=1 / sqrt(queries.shape[-1]))
+            queries, keys, values = (layer(tensor) for layer in (self.query, self.key, self.value))
+            keys, values = cache.update(self._split(keys), self._split(values))
+            batch, length, features = tensor.shape
+            total, dim = keys.shape[2:]
+            stores = tuple(x.storage for x in (queries, keys, values))
+            if matmul_precision() is None and amd_lm.attention_cached_serves(*stores, length, total, dim):
+                mixed = amd_lm.attention_cached(*stores, batch, length, total, self.heads, dim)
+                return self.output(Tensor(mixed, shape=(batch, length, features)))
+            scores = matmul(self._split(queries), keys.transpose((0, 1, 3, 2)))
+            probabilities = softmax(causal_mask(scores, offset=total - length), -1, scale=1 / sqrt(dim))
             mixed = matmul(probabilities, values)
-            batch, _, features = tensor.shape
             return self.output(mixed.transpose((0, 2, 1, 3)).reshape((batch, length, features)))
 
     def parameters(self):
