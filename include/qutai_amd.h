@@ -45,13 +45,15 @@ int qutai_amd_device_arch(int device, char* name, size_t size);
  *   A_z(m,k) = transpose_left  ? a[z*left_stride  + k*rows + m] : a[z*left_stride  + m*inner + k]
  *   B_z(k,n) = transpose_right ? b[z*right_stride + n*inner + k] : b[z*right_stride + k*cols + n]
  * out is [batch][rows][cols] contiguous.  A stride of 0 broadcasts one
- * operand over the batch.  fp32 x fp32 runs on v_mfma_f32_32x32x2_f32; any
- * bf16 operand, or bf16_compute != 0 (autocast), runs on
- * v_mfma_f32_32x32x16_bf16 with fp32 accumulation, an fp32 operand being
- * rounded to bf16 (nearest even) into `workspace` first (see
+ * operand over the batch.  fp32 x fp32 runs on v_mfma_f32_32x32x16_bf16 with
+ * every value as three bf16 parts (all 24 bits, six products each; tiles with
+ * outputs that are not finite or vanish are redone with
+ * v_mfma_f32_32x32x2_f32); any bf16 operand, or bf16_compute != 0 (autocast),
+ * runs on v_mfma_f32_32x32x16_bf16 with fp32 accumulation, an fp32 operand
+ * being rounded to bf16 (nearest even) into `workspace` first (see
  * qutai_amd_gemm_workspace_size for when a workspace is needed and how
- * large); fp64 runs a SIMT
- * kernel.  accumulate != 0 adds the old output before the single rounding
+ * large); fp64 runs a SIMT kernel.  accumulate != 0 adds the old output before
+ * the single rounding
  * to out_dtype.  inner == 0 writes zeros (or keeps out when accumulating).
  * Replaces: `cuda.gemm` (src/qutai/backends/cuda.py:305-362) and the kernels
  * gemm_tiled / gemm_register / gemm_bf16 / gemm_bf16_wide / gemm_bf16_long
@@ -67,9 +69,11 @@ int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_
  * array in device memory of qutai_amd_gemm_static_capacity() bytes
  * (128 MiB) per GPU, held by the library until the process ends; the
  * caller still passes inputs and output.  Results are bit-identical to
- * qutai_amd_gemm (same kernels).  Returns QA_ESCRATCH when the operands need
- * more workspace than that (e.g. fp32 operands into the bf16 path of more
- * than 64 Mi elements together), before launching anything.  Every call on
+ * qutai_amd_gemm (same kernels), except where the partial sums of K chunks do
+ * not fit beside the operands' re-layouts: that product runs in one piece.
+ * Returns QA_ESCRATCH when the re-layouts themselves need more than that (e.g.
+ * fp32 operands into the bf16 path of more than 64 Mi elements together),
+ * before launching anything.  Every call on
  * one GPU shares that GPU's array, so calls that overlap on one GPU (two
  * streams, two host threads) race; calls in one stream are ordered.
  * No counterpart in the reference: for callers that cannot allocate device

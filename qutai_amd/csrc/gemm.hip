@@ -923,10 +923,17 @@ size_t qutai_amd_gemm_workspace_size(int64_t rows, int64_t inner, int64_t cols, 
   return (pa.copy ? pa.bytes : 0) + (pb.copy ? pb.bytes : 0) + partial + 256;
 }
 
-int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_t inner, int64_t cols,
+}  // extern "C"
+
+namespace qa {
+
+// A plain product.  With `spare`, K chunks whose partial sums do not fit beside
+// the operands' re-layouts are given up for the product in one piece (the
+// caller's workspace is fixed); without, a small workspace is an error.
+int gemm_plain(const void* a, const void* b, void* out, int64_t rows, int64_t inner, int64_t cols,
                    int64_t batch, int64_t left_stride, int64_t right_stride, int transpose_left,
                    int transpose_right, int a_dtype, int b_dtype, int out_dtype, int accumulate,
-                   int bf16_compute, void* workspace, size_t workspace_bytes, void* stream_) {
+                   int bf16_compute, void* workspace, size_t workspace_bytes, bool spare, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
   if (rows < 0 || inner < 0 || cols < 0 || batch < 0 || left_stride < 0 || right_stride < 0) return QA_EINVAL;
   bool f64 = a_dtype == QA_F64 || b_dtype == QA_F64;
@@ -955,6 +962,15 @@ int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_
   const int count = plan_windows(rows, inner, cols, batch, bf16, transpose_left, w);
   size_t partial = 0;
   for (int i = 0; i < count; i++) partial += w[i].partial;
+  if (spare && partial && workspace_bytes < (pa.copy ? pa.bytes : 0) + (pb.copy ? pb.bytes : 0) + partial + 256) {
+    partial = 0;
+    for (int i = 0; i < count; i++)
+      if (w[i].partial) {
+        w[i].tile = choose_tile(rows, w[i].n, inner, batch, bf16, transpose_left);
+        w[i].splits = 1;
+        w[i].partial = 0;
+      }
+  }
   char* part = nullptr;
   // the column remainder's arguments: A as planned (re-laid out before it
   // runs), B's r columns from column c0 of `b_ptr` (row pitch ldb_src)
@@ -1080,6 +1096,18 @@ int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_
     if (err != hipSuccess) return (int)err;
   }
   return QA_OK;
+}
+
+}  // namespace qa
+
+extern "C" {
+
+int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_t inner, int64_t cols,
+                   int64_t batch, int64_t left_stride, int64_t right_stride, int transpose_left,
+                   int transpose_right, int a_dtype, int b_dtype, int out_dtype, int accumulate,
+                   int bf16_compute, void* workspace, size_t workspace_bytes, void* stream_) {
+  return qa::gemm_plain(a, b, out, rows, inner, cols, batch, left_stride, right_stride, transpose_left, transpose_right,
+                    a_dtype, b_dtype, out_dtype, accumulate, bf16_compute, workspace, workspace_bytes, false, stream_);
 }
 
 int qutai_amd_gemm_grouped(const void* a, const void* b, void* out, const int64_t* offsets, int groups,

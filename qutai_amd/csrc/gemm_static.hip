@@ -9,6 +9,13 @@
 
 #include "qutai_amd.h"
 
+namespace qa {  // gemm.hip
+int gemm_plain(const void* a, const void* b, void* out, int64_t rows, int64_t inner, int64_t cols, int64_t batch,
+               int64_t left_stride, int64_t right_stride, int transpose_left, int transpose_right, int a_dtype,
+               int b_dtype, int out_dtype, int accumulate, int bf16_compute, void* workspace, size_t workspace_bytes,
+               bool spare, void* stream);
+}  // namespace qa
+
 namespace {
 
 constexpr size_t SCRATCH_BYTES = (size_t)128 << 20;
@@ -59,15 +66,15 @@ int qutai_amd_gemm_static(const void* a, const void* b, void* out, int64_t rows,
     return qutai_amd_gemm(a, b, out, rows, inner, cols, batch, left_stride, right_stride, transpose_left,
                           transpose_right, a_dtype, b_dtype, out_dtype, accumulate, bf16_compute, nullptr, 0,
                           stream);
-  if (need > SCRATCH_BYTES) return QA_ESCRATCH;
   void* ptr = nullptr;
   const int status = scratch_address(&ptr);
   if (status != QA_OK) return status;
-  // qutai_amd_gemm checks the exact need (incl. a misaligned base) against
-  // the capacity and returns QA_EWORKSPACE when it does not fit
-  const int result = qutai_amd_gemm(a, b, out, rows, inner, cols, batch, left_stride, right_stride, transpose_left,
+  // the exact need (incl. a misaligned base) is checked against the capacity
+  // before any launch: partial sums that do not fit are done without,
+  // re-layouts that do not fit are QA_EWORKSPACE
+  const int result = qa::gemm_plain(a, b, out, rows, inner, cols, batch, left_stride, right_stride, transpose_left,
                                     transpose_right, a_dtype, b_dtype, out_dtype, accumulate, bf16_compute, ptr,
-                                    SCRATCH_BYTES, stream);
+                                    SCRATCH_BYTES, true, stream);
   return result == QA_EWORKSPACE ? QA_ESCRATCH : result;
 }
 

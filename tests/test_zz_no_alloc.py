@@ -99,3 +99,18 @@ def test_oversized_request_is_refused_before_launch(amd):
     small = static_gemm(amd, amd.full(64 * 64, 1.0, dtype="float32"), amd.full(64 * 64, 2.0, dtype="float32"), 64,
                         64, 64, bf16_compute=True)
     assert (download(small) == 128.0).all()
+
+
+def test_partial_sums_that_do_not_fit_beside_the_copies(amd):
+    """Re-layouts of 122 MiB (rows of 4001 values) leave no room for the
+    partial sums of K chunks: the product runs in one piece."""
+    rows, inner, cols = 8000, 4001, 128
+    need = amd.get_runtime().gemm_workspace(rows, inner, cols, 1, rows * inner, inner * cols, 0, 0, 0, 0, 0)
+    copies = rows * 4004 * 4
+    assert copies < 128 << 20 < need, "the sizes no longer reach the limit"
+    w = normal(300, (inner, cols))
+    a, b = amd.full(rows * inner, 1.0, dtype="float32"), upload(w, "float32")
+    got = np.asarray(download(static_gemm(amd, a, b, rows, inner, cols))).reshape(rows, cols)
+    wide = np.asarray(w, dtype=np.float32).astype(np.float64)
+    bound = inner * 2.0 ** -24 * np.abs(wide).sum(axis=0)  # a rounded add per term
+    assert (np.abs(got - wide.sum(axis=0)) <= bound).all()
