@@ -410,6 +410,13 @@ int qutai_amd_attention_fwd(const void* q, const void* k, const void* v, void* o
 int qutai_amd_attention_cached(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t heads,
                                int64_t length, int64_t total, int64_t dim, int dtype, double scale, void* stream);
 
+/* A key and a value cache extended in one launch: out[r] = past[r] followed by
+ * new[r] for each of `rows` (batch, head) rows of past_bytes and new_bytes, both
+ * multiples of 16, all pointers 16-byte aligned; out does not overlap the
+ * inputs.  Replaces the concatenations of src/qutai/nn/cache.py:5-29. */
+int qutai_amd_cache_join(const void* past_k, const void* past_v, const void* new_k, const void* new_v, void* out_k,
+                         void* out_v, int64_t rows, int64_t past_bytes, int64_t new_bytes, void* stream);
+
 /* Grouped-K GEMM for the MoE weight gradients: for every group g,
  *   out[g] (rows x cols) (+)= A_g^T B_g,
  * where A_g / B_g are the K rows [offsets[g], offsets[g+1]) of a ([K][rows])

@@ -499,6 +499,24 @@ def attention_cached(q, k, v, batch, length, total, heads, dim):
     return out
 
 
+def cache_join(past, new, rows):
+    """(keys, values) of earlier positions followed by new ones in each of
+    ``rows`` (batch, head) rows, in one launch (src/qutai/nn/cache.py:5-29);
+    None where rows are not whole 16-byte chunks of one type."""
+    stores = (*past, *new)
+    dtype, item = past[0].dtype, amd._item(past[0].dtype)
+    if not rows or any(x.dtype != dtype or x.ptr % 16 for x in stores) or past[0].size != past[1].size \
+            or new[0].size != new[1].size or any(x.size % rows or x.size // rows * item % 16 for x in stores):
+        return None
+    past_bytes, new_bytes = past[0].size // rows * item, new[0].size // rows * item
+    # the launch holds 2 x rows x (16 KiB segments of a row) workgroups
+    if not new_bytes or max(past_bytes, new_bytes) > 1 << 34 or rows * ((past_bytes + new_bytes >> 14) + 1) > 1 << 29:
+        return None
+    out = tuple(AMDStorage(past[0].size + new[0].size, dtype) for _ in range(2))
+    out[0].runtime.call("qutai_amd_cache_join", *(x.ptr for x in (*stores, *out)), rows, past_bytes, new_bytes)
+    return out
+
+
 def attention_backward(gradient, q, k, v, out, lse, batch, time, heads, kv_heads, dim, *, causal=True, layout=1,
                        scale=None):
     """(dq, dk, dv) of ``attention`` (cuda_lm.attention_backward,

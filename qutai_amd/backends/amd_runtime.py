@@ -81,6 +81,7 @@ SIGNATURES = {
     "qutai_amd_head_gradient": [_p, _p, _p, _i64, _i64, _f64, _i32, _p],
     "qutai_amd_attention_fwd": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _f64, _i32, _p],
     "qutai_amd_attention_cached": [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i32, _f64, _p],
+    "qutai_amd_cache_join": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p],
     "qutai_amd_attention_bwd": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i64, _i64, _i64, _i64, _i64, _i32,
                                 _i32, _f64, _i32, _p],
     "qutai_amd_attention_bwd_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i32],

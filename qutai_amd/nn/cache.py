@@ -2,12 +2,14 @@
 (src/qutai/nn/cache.py:5-29).
 
 The cache holds (batch, heads, length, head_dim) tensors with no graph:
-``update`` appends the new positions along the length axis (one strided
+``update`` appends the new positions along the length axis (keys and values
+in one launch where their rows are whole 16-byte chunks, else one strided
 copy per piece through ``backend.concatenate``) and returns everything
 cached so far.
 """
 from __future__ import annotations
 
+from ..backends import amd_lm
 from ..backends.device import get_backend
 from ..core.tensor import Tensor
 
@@ -38,5 +40,13 @@ class KVCache:
         if self.keys is not None and (self.keys.shape[:2] + self.keys.shape[3:]
                                       != keys.shape[:2] + keys.shape[3:]):
             raise ValueError("new keys and values must match the cache in batch, heads and head size")
+        if self.keys is not None and self.keys.shape == self.values.shape:
+            batch, heads, past, features = self.keys.shape
+            joined = amd_lm.cache_join((self.keys.storage, self.values.storage), (keys.storage, values.storage),
+                                       batch * heads)
+            if joined is not None:
+                shape = (batch, heads, past + keys.shape[2], features)
+                self.keys, self.values = (Tensor(x, shape=shape) for x in joined)
+                return self.keys, self.values
         self.keys, self.values = _joined(self.keys, keys), _joined(self.values, values)
         return self.keys, self.values

@@ -5,7 +5,9 @@ import numpy as np
 import pytest
 
 from oracle import reference as ora
+from qutai_amd import Tensor
 from qutai_amd.backends import amd, amd_lm
+from qutai_amd.nn import KVCache
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +67,20 @@ def test_cached_attention_refuses_what_its_kernel_cannot_hold():
             amd_lm.attention_cached(one, one, one, 1, length, total, 1, dim)
     with pytest.raises(ValueError):
         amd_lm.attention_cached(one, one, one, 1, 1, 11, 1, 8)
+
+
+@pytest.mark.parametrize("dtype,batch,heads,past,new,dim", [
+    ("bfloat16", 1, 1, 1, 1, 8), ("float32", 3, 5, 7, 2, 12), ("bfloat16", 2, 3, 127, 1, 64),
+    ("float32", 2, 2, 1023, 2, 4), ("bfloat16", 2, 2, 300, 70, 128), ("float32", 1, 3, 5, 2, 6), ("bfloat16", 1, 2, 3, 1, 20),
+])
+def test_cache_update_joins_keys_and_values(dtype, batch, heads, past, new, dim):
+    """Rows of one chunk, around one and two segments of 1024 chunks, new positions
+    longer than a workgroup's stride; the last two take the copies."""
+    rng = np.random.default_rng(past)
+    old, fresh = ([_draw(rng, (batch, heads, n, dim), dtype) for _ in range(2)] for n in (past, new))
+    cache = KVCache()
+    for pair in (old, fresh):
+        got = cache.update(*(Tensor(amd.storage(x.ravel().tolist(), dtype=dtype), shape=x.shape) for x in pair))
+    for x, a, b in zip(got, old, fresh):
+        assert x.shape == (batch, heads, past + new, dim)
+        assert np.array_equal(np.array(x.storage.tolist()).reshape(x.shape), np.concatenate((a, b), 2))
