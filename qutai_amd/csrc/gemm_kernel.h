@@ -212,9 +212,11 @@ struct GemmKernel {
   // matrix gets an offset beyond the descriptor's range, for which the
   // hardware returns zeros.  Operands whose rows are not 16-byte aligned are
   // re-laid out (zero-padded pitch) by the host entry point before the launch.
+  // OOB is outside every range: a range is never negative (an unsigned
+  // length that wrapped would hold it) and at most 0x7ffffff0.
   static constexpr uint32_t OOB = 0x80000000u;
   __device__ static __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const T* base, int64_t bytes) {
-    uint32_t n = bytes > 0x7ffffff0 ? 0x7ffffff0u : (uint32_t)bytes;
+    const uint32_t n = bytes <= 0 ? 0u : bytes > 0x7ffffff0 ? 0x7ffffff0u : (uint32_t)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, n, 0x00020000);
   }
   __device__ static __forceinline__ u32x4 fetch16(__amdgpu_buffer_rsrc_t r, uint32_t offset) {
@@ -438,13 +440,16 @@ struct GemmKernel {
       const T* a = tail ? w.a_tail : w.a;
       const T* b = tail ? w.b_tail : w.b;
       // bases as in run()'s ring: A from its first row (gathered rows: the
-      // whole matrix), B from its first column
-      const auto da = w.a_rows ? rsrc(a + ks, w.a_bytes - ks * 4)
+      // whole matrix), B from its first column.  A stage past K, which the
+      // lookahead of small tiles asks for, has empty descriptors: it reads
+      // zeros and touches no memory.
+      const bool some = k0 < w.K;
+      const auto da = w.a_rows ? rsrc(a + ks, some ? w.a_bytes - ks * 4 : 0)
                                : rsrc(KA ? a + w.row0 * w.lda + ks : a + ks * w.lda + w.row0,
-                                      (KA ? BM * w.lda : 16 * w.lda) * 4);
-      const auto db = GATHER_B ? rsrc(b + w.col0, w.b_bytes - w.col0 * 4)
+                                      some ? (KA ? BM * w.lda : 16 * w.lda) * 4 : 0);
+      const auto db = GATHER_B ? rsrc(b + w.col0, some ? w.b_bytes - w.col0 * 4 : 0)
                                : rsrc(KB ? b + w.col0 * w.ldb + ks : b + ks * w.ldb + w.col0,
-                                      (KB ? BN * w.ldb : 16 * w.ldb) * 4);
+                                      some ? (KB ? BN * w.ldb : 16 * w.ldb) * 4 : 0);
       const int64_t krem = w.K - k0;
 #pragma unroll
       for (int j = 0; j < ITEMS; j++) {

@@ -12,13 +12,12 @@ compute -- per tile, K step, copy instruction and lane -- so that tests can
 check over randomised shapes that every issued load and every store lies
 inside its allocation.
 
-Restated from qutai_amd/csrc/gemm_kernel.h (tile scheduling and operand
-bases 342-404, descriptor bases 418-425 and 466-471, DMA lane offsets
-430-465, register-staging offsets 523-545, epilogue 590-660 and 711-770) and
-qutai_amd/csrc/gemm_short.h (copies 91-101, output offsets 104-112 and
-176-186); the host's operand re-layout rule (plan_operand), split-K chunking
-(choose_split), grouped grid and the pair form's K join from
-qutai_amd/csrc/gemm.hip.
+Restated from qutai_amd/csrc/gemm_kernel.h (run's tile scheduling, operand and
+descriptor bases, copy and register-staging offsets and epilogue; reduce_parts,
+which every fp32 product runs first: its items, the stages it fetches past K and
+its descriptors) and qutai_amd/csrc/gemm_short.h (copies and output offsets); the
+host's operand re-layout rule (plan_operand), split-K chunking (choose_split),
+grouped grid and the pair form's K join from qutai_amd/csrc/gemm.hip.
 """
 from __future__ import annotations
 
@@ -52,7 +51,9 @@ def tile_configs(f32: bool) -> list[Config]:
     table = [Config("L8D2", 256, 256, 2, 4, kr, 2), Config("L8R", 256, 256, 2, 4, kr, 2, dma=False),
              Config("L4D2", 256, 256, 2, 2, kr, 2), Config("S", 128, 128, 2, 2, kb, 4),
              Config("S2", 128, 128, 2, 2, kb, 2), Config("N", 256, 64, 4, 1, kr, 2),
-             Config("W", 64, 256, 1, 4, kb, 4), Config("H", 256, 128, 4, 2, kr, 3)]
+             Config("W", 64, 256, 1, 4, kb, 4), Config("H", 256, 128, 4, 2, kr, 3),
+             Config("X", 128, 128, 2, 4, kr, 2 if f32 else 3), Config("Y", 128, 64, 2, 2, kb if f32 else kr, 3),
+             Config("Z", 64, 64, 2, 2, kb if f32 else kr, 3)]
     if f32:
         table += [Config("T", 256, 256, 2, 4, kr, 2), Config("U", 256, 256, 2, 4, kr, 2)]
     else:
@@ -108,6 +109,84 @@ def _check(what: str, lo: np.ndarray, hi: np.ndarray, alloc_bytes: int):
     if lo.min() < 0 or hi.max() > alloc_bytes:
         bad = np.flatnonzero((lo < 0) | (hi > alloc_bytes))[0]
         raise Violation(f"{what}: access [{lo.flat[bad]}, {hi.flat[bad]}) outside [0, {alloc_bytes})")
+
+
+def records(nbytes: int, clamped: bool = True) -> int:
+    """The range of a descriptor as the hardware holds it: 32 bits.  Without
+    the clamp at zero -- a planted mistake -- a negative length wraps."""
+    if nbytes > RANGE_CAP:
+        return RANGE_CAP
+    return max(nbytes, 0) if clamped else nbytes & 0xFFFFFFFF
+
+
+def part_stages(cfg: Config, k_len: int) -> list[int]:
+    """First k of every stage (16 of K) that reduce_parts fetches: one stage
+    ahead on 256x256 tiles, which skip stages past the next; two on smaller
+    ones, whose steps come in pairs and fetch without a condition."""
+    depth = 1 if cfg.bm * cfg.bn >= 256 * 256 else 2
+    nk = (k_len + 15) // 16
+    steps = [kt for kt in range(nk) if kt + 1 < nk] if depth == 1 else range(nk + nk % 2)
+    return [16 * s for s in sorted({*range(depth + 1), *(kt + 1 + depth for kt in steps)})]
+
+
+def part_loads(cfg: Config, kmajor: bool, rows_tile: int, base_elem: int, row0: int, rows: int, k_len: int, ld: int,
+               alloc: int, what: str, gather: np.ndarray | None = None, empty_past_k: bool = True):
+    """reduce_parts' loads of one fp32 operand: items of eight elements, two
+    16-byte loads each.  empty_past_k False -- a planted mistake -- keeps the
+    descriptors of stages past K as they would follow from k0, unclamped."""
+    q = np.arange(2 * rows_tile)
+    per = rows_tile // 8
+    outer, c = (q >> 1, q & 1) if kmajor else (q // per, q % per)
+    kk = 8 * c if kmajor else outer
+    src = outer
+    inside = [row0 + (outer if kmajor else 8 * c + 4 * half) < rows for half in (0, 1)]
+    if gather is not None:
+        src = np.where(inside[0], gather[np.minimum(row0 + outer, gather.size - 1)], outer)
+        known = (src >= 0) & (src < alloc // ld)
+        inside = [x & known for x in inside]
+    off = ((src * ld + 8 * c) * 4) & 0xFFFFFFFF
+    for k0 in part_stages(cfg, k_len):
+        if gather is not None:
+            tile_elem, span = base_elem + k0, alloc * 4 - k0 * 4
+        else:
+            tile_elem = base_elem + (row0 * ld + k0 if kmajor else k0 * ld + row0)
+            span = (rows_tile if kmajor else 16) * ld * 4
+        n = records(0 if empty_past_k and k0 >= k_len else span, empty_past_k)
+        for half in (0, 1):
+            issued = inside[half] & (kk + (4 * half if kmajor else 0) < k_len - k0)
+            offs = np.where(issued, off + 16 * half, OOB)
+            hit = offs + 16 <= n
+            if np.any(issued & ~hit):
+                raise Violation(f"{what} (parts): an in-matrix chunk falls outside the descriptor range")
+            lo = tile_elem * 4 + offs[hit]
+            _check(f"{what} load (parts)", lo, lo + 16, alloc * 4)
+
+
+def part_loads_gathered_k(cfg: Config, col0: int, cols: int, k_lo: int, k_len: int, gather: np.ndarray,
+                          source_rows: int, empty_past_k: bool = True):
+    """reduce_parts' loads of an MN-major B whose K rows are gathered."""
+    alloc = source_rows * cols
+    q = np.arange(2 * cfg.bn)
+    outer, c = q // (cfg.bn // 8), q % (cfg.bn // 8)
+    for k0 in part_stages(cfg, k_len):
+        n = records(0 if empty_past_k and k0 >= k_len else alloc * 4 - col0 * 4, empty_past_k)
+        k = k0 + outer
+        read = (col0 + 8 * c < cols) & (k < k_len)
+        at = k_lo + k[read]
+        if at.size and (at.min() < 0 or at.max() >= gather.size):
+            raise Violation("B (parts): an index read outside the route order")
+        src = np.full(q.size, -1, dtype=np.int64)
+        src[read] = gather[at]
+        known = (src >= 0) & (src < source_rows)
+        off = ((src * cols + 8 * c) * 4) & 0xFFFFFFFF
+        for half in (0, 1):
+            issued = known & (col0 + 8 * c + 4 * half < cols) & (k < k_len)
+            offs = np.where(issued, off + 16 * half, OOB)
+            hit = offs + 16 <= n
+            if np.any(issued & ~hit):
+                raise Violation("B (parts, gathered): an in-matrix chunk falls outside the descriptor range")
+            lo = col0 * 4 + offs[hit]
+            _check("B (parts, gathered) load", lo, lo + 16, alloc * 4)
 
 
 def operand_loads(cfg: Config, f32: bool, kmajor: bool, rows_tile: int, base_elem: int, row0: int, rows: int,
@@ -377,6 +456,8 @@ def gathered_k_loads(cfg: Config, f32: bool, col0: int, cols: int, k_lo: int, k_
     if cfg.stages != 2 or not cfg.dma:
         raise ValueError("gathered K rows run on the two-stage direct-to-LDS tiles only")
     alloc = source_rows * cols
+    if f32:
+        part_loads_gathered_k(cfg, col0, cols, k_lo, k_len, gather, source_rows)
     q = np.arange(cfg.bn * cfg.bk // e)
     outer, c = chunk_coords(f32, False, cfg.bn, cfg.bk, q)
     valid = col0 + c * e < cols

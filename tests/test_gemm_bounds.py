@@ -198,6 +198,36 @@ def test_model_reports_a_gathered_k_index_past_the_source():
         gm.grouped_k_gemm(cfg, False, [3, 0, 5], 16, 64, gather=order, source_rows=8, index_check=False)
 
 
+@pytest.mark.parametrize("tile", ["X", "Z", "L8D2"])
+def test_fp32_parts_of_few_rows_stay_in_bounds(tile):
+    """fp32 products of one to four gathered rows, whose operand is shorter
+    than the stages that are fetched past K, and an empty source."""
+    cfg = next(c for c in gm.tile_configs(True) if c.name == tile)
+    for tokens in (1, 2, 4):
+        order = np.tile(np.arange(tokens), 2)
+        for inner in (4, 8, 20, 64, 100, 1024):
+            gm.grouped_gemm(cfg, True, [tokens, 0, tokens], inner, 40, True, gather=order, source_rows=tokens)
+            gm.grouped_gemm(cfg, True, [tokens, tokens], inner, 40, False)
+            gm.grouped_k_gemm(next(c for c in gm.tile_configs(True) if c.name == "L8D2"), True, [tokens, 0, tokens],
+                              inner, 36, gather=order, source_rows=tokens)
+    gm.part_loads_gathered_k(cfg, 128, 256, 0, 0, np.zeros(0, dtype=np.int64), 0)
+
+
+def test_model_reports_stages_past_k_with_a_wrapped_range():
+    """A planted mistake: the descriptor of one gathered row of 1024 moves on
+    with k0 past K, its length goes below zero and wraps to nearly 4 GiB, and
+    the offset of masked loads, 2 GiB, is inside it.  The same with an odd K on
+    the 256x256 tile, and with an empty gathered B from column 128 on."""
+    one = np.zeros(2, dtype=np.int64)
+    tiles = {c.name: c for c in gm.tile_configs(True)}
+    for tile, k in (("Z", 1024), ("X", 40), ("L8D2", 20)):
+        gm.part_loads(tiles[tile], True, tiles[tile].bm, 0, 0, 1, k, k, k, "A", one)
+        with pytest.raises(gm.Violation):
+            gm.part_loads(tiles[tile], True, tiles[tile].bm, 0, 0, 1, k, k, k, "A", one, empty_past_k=False)
+    with pytest.raises(gm.Violation):
+        gm.part_loads_gathered_k(tiles["Z"], 128, 256, 0, 0, np.zeros(0, dtype=np.int64), 0, empty_past_k=False)
+
+
 def test_short_k_strips_stay_in_bounds():
     rng = np.random.default_rng(SEED + 17)
     for m, k, n, batch in [(700, 64, 1040, 2), (129, 24, 144, 3), (64, 8, 2064, 1), (2048, 64, 256, 1)]:

@@ -174,6 +174,32 @@ def test_sparse_moe_layer_forward_and_all_gradients(lm):
     assert sum(layer.last_counts) == tokens * top_k
 
 
+@pytest.mark.parametrize("tokens,width,hidden", [(1, 1024, 64), (2, 1024, 64), (1, 8, 24), (2, 8, 20), (4, 8, 24),
+                                                 (3, 20, 12)])
+def test_sparse_moe_of_a_few_tokens(lm, tokens, width, hidden):
+    """fp32 expert products over gathered rows of an operand that is shorter
+    than the K stages the kernel looks ahead (one token of a generation step)."""
+    from qutai_amd import Tensor
+    from qutai_amd.lm.layers import SparseMoE
+
+    experts, top_k = 4, 2
+    layer = SparseMoE(width, hidden, experts, top_k, seed=tokens)
+    xv, G = normal(tokens, tokens * width), normal(width, tokens * width)
+    x = Tensor(upload(xv, "float32"), shape=(tokens, width), requires_grad=True)
+    y, _ = layer(x)
+    y.backward(Tensor(upload(G, "float32"), shape=y.shape))
+    f64 = lambda t, shape: download(t.storage).astype(np.float64).reshape(shape)  # noqa: E731
+    parameters = (layer.router.weight, layer.w_gate, layer.w_up, layer.w_down)
+    shapes = ((experts, width), (experts, hidden, width), (experts, hidden, width), (experts, width, hidden))
+    ry, _, rdx, *grads = moe_reference(xv.reshape(tokens, width).astype(np.float64),
+                                       *(f64(p, s) for p, s in zip(parameters, shapes)), top_k,
+                                       G.reshape(tokens, width).astype(np.float64), 0.0)
+    assert ora.rel_frobenius(f64(y, ry.shape), ry) <= 2e-5
+    assert ora.rel_frobenius(f64(x.grad, rdx.shape), rdx) <= 2e-5
+    for p, s, expected in zip(parameters, shapes, grads):
+        assert ora.rel_frobenius(f64(p.grad, s), expected) <= 2e-5
+
+
 @pytest.mark.parametrize("dtype,width,hidden", [("bfloat16", 256, 200), ("float32", 256, 200),
                                                 ("bfloat16", 36, 20)])
 def test_backward_through_the_order_equals_the_gathered_copy(lm, dtype, width, hidden):
