@@ -47,7 +47,7 @@ int qutai_amd_device_arch(int device, char* name, size_t size);
  * out is [batch][rows][cols] contiguous.  A stride of 0 broadcasts one
  * operand over the batch.  fp32 x fp32 runs on v_mfma_f32_32x32x16_bf16 with
  * every value as three bf16 parts (all 24 bits, six products each; tiles with
- * outputs that are not finite or vanish are redone with
+ * values from 2^103 or sums from 2^80 on, infinities or NaN are redone with
  * v_mfma_f32_32x32x2_f32); any bf16 operand, or bf16_compute != 0 (autocast),
  * runs on v_mfma_f32_32x32x16_bf16 with fp32 accumulation, an fp32 operand
  * being rounded to bf16 (nearest even) into `workspace` first (see

@@ -380,12 +380,14 @@ struct GemmKernel {
   // Bound by the MFMAs at the power limit for whole rounds of 256x256 tiles
   // (4096^3: 976 us with the fp32 MFMA, 666 now, 60% of the MFMA cycles); by
   // the latency of a stage with one wave per SIMD on small tiles.
-  // An infinity or NaN has parts whose products give NaN, so it shows in the
-  // accumulators.  An element below 2^-110 loses up to 2^-134 (bf16's
-  // smallest step): with every output above 2^-80 that is below fp32's own
-  // rounding as long as the elements it meets are below 2^30 / K.  Returns
-  // whether this thread's outputs are all zero or finite and above 2^-80; a
-  // tile with one that is not is computed again with the fp32 MFMA.
+  // Operands are split as 2^24 of their values, and the sums come back as 2^-48
+  // of theirs: the 24 bits of every finite value, subnormals included, then end
+  // above bf16's smallest normal (2^-149 as 2^-125), and no term that fp32 can
+  // hold falls below the MFMA's range.  Both factors sit in operations that the
+  // alternating sign needs anyway.  A value from 2^103 on, 16 products above
+  // 2^80, an infinity or NaN has parts or sums that are not finite, which shows
+  // in the accumulators.  Returns whether this thread's outputs are all finite;
+  // a tile with one that is not is computed again with the fp32 MFMA.
   __device__ static __forceinline__ bool reduce_parts(const Work& w, char* smem, f32x16 (&acc)[FM][FN], int tid) {
     constexpr int NA = 2 * BM, ITEMS = (2 * (BM + BN) + NT - 1) / NT;  // eight-element items: A's, then B's
     const int lane = tid & 63, wave = uniform32(tid >> 6), wm = wave / WN, wn = wave % WN;
@@ -466,13 +468,14 @@ struct GemmKernel {
         raw[slot][j][1] = fetch16(is_a ? da : db, ok && in[j][1] && kk[j] + (kmajor ? 4 : 0) < krem ? o + 16 : OOB);
       }
     };
-    // the fetched stage into its planes; A times `sign`
+    constexpr float UP = 0x1p24f, DOWN = 0x1p-48f;
+    // the fetched stage into its planes, times UP; A times `sign` too
     auto put = [&](int slot, int stage, float sign) {
 #pragma unroll
       for (int j = 0; j < ITEMS; j++) {
         if (wave * 64 + j * NT >= 2 * (BM + BN)) continue;
         const bool is_a = wave * 64 + j * NT < NA;
-        const float f = is_a ? sign : 1.f;
+        const float f = is_a ? sign * UP : UP;
         float v[8];
         bf16x8 part[3];
 #pragma unroll
@@ -536,7 +539,9 @@ struct GemmKernel {
             for (int j = 0; j < FN; j++)
               sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[x], pb[j][order - x], sum[j], 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] += sum[j] * sign;
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[i][j][e] = __builtin_fmaf(sum[j][e], sign * DOWN, acc[i][j][e]);
       }
       if constexpr (!BIG) {
         // per MFMA: one LDS read, a share of the split and the adds, one LDS write
@@ -570,10 +575,7 @@ struct GemmKernel {
 #pragma unroll
       for (int j = 0; j < FN; j++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-          const float x = __builtin_fabsf(acc[i][j][e]);
-          fine &= (x < INFINITY) & (x >= 0x1p-80f | x == 0.f);
-        }
+        for (int e = 0; e < 16; e++) fine &= __builtin_fabsf(acc[i][j][e]) < INFINITY;
     return fine;
   }
 

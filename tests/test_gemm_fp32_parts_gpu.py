@@ -45,6 +45,23 @@ def test_subnormal_operands_keep_their_bits(amd):
     assert ora.rel_frobenius(product(amd, a, b), exact) <= 2e-6
 
 
+# Each product of two values takes three bf16 parts of each: all of them count,
+# whatever the two magnitudes are, and the sum rounds as fp32 sums do.  Where
+# outputs are subnormal they round to 2^-149, whose share of the smallest rms
+# here (1e-38 sqrt(40)) is below 1e-7.
+@pytest.mark.parametrize("small,large", [(1e-41, 1e35), (1e-41, 1e3), (3e-39, 1e20), (3e-39, 1e5), (1e-36, 1.0),
+                                         (1e-33, 1e30), (1e-20, 1e-18), (1e-30, 1e30), (1e25, 1e11), (1e-45, 1e24)])
+@pytest.mark.parametrize("m,k,n", [(96, 40, 160), (300, 500, 280)])
+def test_far_apart_magnitudes(amd, m, k, n, small, large):
+    a, b = normal(m, (m, k), small), normal(n, (k, n), large)
+    a[5] = 0  # a row of zeros stays one
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    for left, right, expected in ((a, b, exact), (b.T.copy(), a.T.copy(), exact.T)):
+        got = product(amd, left, right)
+        assert ora.rel_frobenius(got, expected) <= 2e-6
+    assert not product(amd, a, b)[5].any()
+
+
 def test_infinities_nan_and_the_top_of_the_range(amd):
     a, b = normal(3, (300, 64)), normal(4, (64, 300))
     a[5, 7], a[9, 3], b[11, 13] = np.inf, np.nan, -np.inf
