@@ -62,6 +62,18 @@ def test_far_apart_magnitudes(amd, m, k, n, small, large):
     assert not product(amd, a, b)[5].any()
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
+def test_one_and_two_products_round_as_fp32_does(amd, ta, tb):
+    """K = 1: the rounded product itself.  K = 2: at most one rounding of each
+    product and one of their sum, half a step (2^-24 of the value) each."""
+    a, b = normal(8, (300, 1)), normal(9, (1, 260))
+    assert np.array_equal(product(amd, a, b, ta, tb), a * b)
+    a, b = normal(10, (300, 2)), normal(11, (2, 260))
+    first, second = (a[:, i:i + 1].astype(np.float64) * b[i:i + 1] for i in (0, 1))
+    bound = 2.0 ** -24 * (np.abs(first) + np.abs(second) + np.abs(first + second)) * (1 + 2.0 ** -23)
+    assert np.all(np.abs(product(amd, a, b, ta, tb) - (first + second)) <= bound)
+
+
 def test_infinities_nan_and_the_top_of_the_range(amd):
     a, b = normal(3, (300, 64)), normal(4, (64, 300))
     a[5, 7], a[9, 3], b[11, 13] = np.inf, np.nan, -np.inf
