@@ -16,18 +16,15 @@ def record(result, parents, rule=None):
 
 def owned(storage):
     """Mark a gradient storage that its backward rule has just allocated and
-    hands to no one else: the leaf that receives it first may keep it as its
-    ``grad`` instead of copying it (the copy isolates storages a rule passes
-    on to several tensors).  Returns the storage; None passes through."""
+    hands to no one else: a leaf that receives it from the rule may keep it as
+    its ``grad`` instead of copying it (the copy isolates storages a rule
+    passes on to several tensors).  ``backward`` drops the mark from a storage
+    that does not go straight to a leaf: one that flows on through other rules
+    or is returned may be passed to several tensors later.  Returns the
+    storage; None passes through."""
     if storage is not None:
         storage.owned_gradient = True
     return storage
-
-
-def owned_by_leaf(storage, parent):
-    """``owned`` for a gradient that goes straight to a leaf.  (One that flows
-    on through other rules may be passed to several tensors by them.)"""
-    return owned(storage) if getattr(parent, "backward_rule", None) is None else storage
 
 
 def take_owned(storage):
@@ -125,5 +122,6 @@ def backward(output, gradient, *, retain_graph=True, leaf_sink=None):
                 else:
                     if isinstance(contribution, DeferredGradient):
                         fresh.add(parent)
-                    gradients[parent] = _dense(contribution)
+                    gradients[parent] = contribution = _dense(contribution)
+                    take_owned(contribution)  # it goes on from here, to whatever tensors
     return leaves

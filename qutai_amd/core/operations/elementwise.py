@@ -10,7 +10,7 @@ materialising the broadcast vector; its gradient is the column sum of G.
 from __future__ import annotations
 
 from ...backends.device import get_backend
-from ..grad import owned_by_leaf
+from ..grad import owned
 from ..shape import broadcast_shape
 
 
@@ -41,8 +41,8 @@ def add(left, right):
             rows, cols = layout
             values = backend.add_rows(big.storage, small.storage, rows, cols)
 
-            def bias_rule(g, rows=rows, cols=cols, bias=small, bias_first=bias_first):
-                column_sums = owned_by_leaf(backend.sum_rows(g, rows, cols), bias)
+            def bias_rule(g, rows=rows, cols=cols, bias_first=bias_first):
+                column_sums = owned(backend.sum_rows(g, rows, cols))
                 return (column_sums, g) if bias_first else (g, column_sums)
 
             return values, big.shape, bias_rule

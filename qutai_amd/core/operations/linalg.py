@@ -28,7 +28,7 @@ from math import prod
 
 from ...backends.device import get_backend
 from ...backends.precision import matmul_precision, set_matmul_precision
-from ..grad import owned_by_leaf
+from ..grad import owned
 from ..shape import broadcast_shape
 
 
@@ -70,8 +70,8 @@ class ProductGradient:
         with set_matmul_precision(self.precision):
             backend = get_backend(gradient.device)
             # each is a storage made here that no one else holds
-            d_left = owned_by_leaf(self._left(backend, gradient), self.left) if self.left.requires_grad else None
-            d_right = owned_by_leaf(self._right(backend, gradient), self.right) if self.right.requires_grad else None
+            d_left = owned(self._left(backend, gradient)) if self.left.requires_grad else None
+            d_right = owned(self._right(backend, gradient)) if self.right.requires_grad else None
         return d_left, d_right
 
     def _layout(self):

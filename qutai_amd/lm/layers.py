@@ -19,7 +19,7 @@ from math import prod, sqrt
 from ..backends import amd, amd_lm
 from ..backends.precision import matmul_precision, set_matmul_precision
 from ..core.context import is_recording
-from ..core.grad import DeferredGradient, owned, owned_by_leaf, record
+from ..core.grad import DeferredGradient, owned, record
 from ..core.tensor import Tensor
 
 
@@ -615,8 +615,7 @@ def attention(q, k, v, heads, kv_heads):
     dims = (batch, time, heads, kv_heads, features // heads)
     out, lse = b.attention(q.storage, k.storage, v.storage, *dims)
     return record(Tensor(out, shape=q.shape), (q, k, v),
-                  lambda g: tuple(map(owned_by_leaf, b.attention_backward(g, q.storage, k.storage, v.storage, out, lse,
-                                                                          *dims), (q, k, v))))
+                  lambda g: tuple(map(owned, b.attention_backward(g, q.storage, k.storage, v.storage, out, lse, *dims))))
 
 
 def _stacked_qkv(x, wq, wk, wv):

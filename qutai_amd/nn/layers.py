@@ -27,7 +27,7 @@ from ..backends import amd, amd_lm
 from ..backends.precision import matmul_precision
 from ..core import operations
 from ..core.context import set_recording
-from ..core.grad import owned_by_leaf, record
+from ..core.grad import owned, record
 from ..core.tensor import Tensor, _result, matmul
 from .cache import KVCache  # noqa: F401 - the reference exposes it beside the layers
 
@@ -83,9 +83,8 @@ def _attend(q, k, v, heads, causal):
     dims = (batch, length, heads, heads, features // heads)
     out, lse = amd_lm.attention(q.storage, k.storage, v.storage, *dims, causal=causal, layout=1)
     return record(Tensor(out, shape=q.shape), (q, k, v),
-                  lambda g: tuple(map(owned_by_leaf, amd_lm.attention_backward(g, q.storage, k.storage, v.storage, out, lse,
-                                                                               *dims, causal=causal, layout=1),
-                                      (q, k, v))))
+                  lambda g: tuple(map(owned, amd_lm.attention_backward(g, q.storage, k.storage, v.storage, out, lse,
+                                                                       *dims, causal=causal, layout=1))))
 
 
 class Attention:

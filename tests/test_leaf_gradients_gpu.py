@@ -38,3 +38,19 @@ def test_kept_gradients_are_not_shared():
     layer(z).backward(Tensor(upload(normal(6, 160), "float32"), shape=(1, 10, 16)))
     pointers = [p.grad.storage.ptr for p in (z, *layer.parameters())]
     assert len(set(pointers)) == len(pointers)
+
+
+def test_checkpoint_of_a_sum_with_a_deferred_gradient():
+    """x gets the checkpoint's gradient through the sum and then the Linear's
+    deferred product, which reads that same gradient."""
+    from qutai_amd import Tensor
+    from qutai_amd.lm import activation_checkpoint, layers
+
+    x, weight, w = (Tensor(upload(normal(7 + i, 256), "float32"), shape=(16, 16), requires_grad=True) for i in range(3))
+    s = x + layers.linear(x, weight)
+    g = Tensor(upload(normal(10, 256), "float32"), shape=(16, 16))
+    activation_checkpoint(lambda t: t @ w, s, parameters=(w,)).backward(g)
+    xs, weights, ws, gs = (download(t.storage).astype(np.float64).reshape(16, 16) for t in (x, weight, w, g))
+    ds = gs @ ws.T
+    for got, want in ((x, ds + ds @ weights), (weight, ds.T @ xs), (w, (xs + xs @ weights.T).T @ gs)):
+        assert np.abs(download(got.grad.storage).reshape(16, 16) - want).max() <= 1e-4 * np.abs(want).max()
