@@ -477,8 +477,9 @@ CACHED_LENGTH, CACHED_KEYS, CACHED_BYTES = 8, 12000, 12000 * 128 * 2
 def attention_cached_serves(q, k, v, length, total, dim):
     """Whether ``attention_cached`` takes operands of these sizes and types."""
     step = {"bfloat16": 8, "float32": 4}.get(q.dtype)  # elements of 16 bytes
-    return (step is not None and q.dtype == k.dtype == v.dtype and dim <= 256 and dim % step == 0
+    return (step is not None and q.dtype == k.dtype == v.dtype and 0 < dim <= 256 and dim % step == 0
             and 0 < length <= CACHED_LENGTH and total <= CACHED_KEYS and total * dim * 16 // step <= CACHED_BYTES
+            and q.size // dim < 1 << 22  # a workgroup of 1024 threads each, fewer than 2^32 threads in a launch
             and all(x.ptr % 16 == 0 for x in (q, k, v)))
 
 
@@ -509,8 +510,8 @@ def cache_join(past, new, rows):
             or new[0].size != new[1].size or any(x.size % rows or x.size // rows * item % 16 for x in stores):
         return None
     past_bytes, new_bytes = past[0].size // rows * item, new[0].size // rows * item
-    # the launch holds 2 x rows x (16 KiB segments of a row) workgroups
-    if not new_bytes or max(past_bytes, new_bytes) > 1 << 34 or rows * ((past_bytes + new_bytes >> 14) + 1) > 1 << 29:
+    # the launch holds 2 x rows x (16 KiB segments of a row) workgroups of 256 threads, fewer than 2^32 threads
+    if not new_bytes or max(past_bytes, new_bytes) > 1 << 34 or rows * -(-(past_bytes + new_bytes) >> 14) >= 1 << 23:
         return None
     out = tuple(AMDStorage(past[0].size + new[0].size, dtype) for _ in range(2))
     out[0].runtime.call("qutai_amd_cache_join", *(x.ptr for x in (*stores, *out)), rows, past_bytes, new_bytes)

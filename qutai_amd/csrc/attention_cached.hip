@@ -209,7 +209,8 @@ extern "C" int qutai_amd_attention_cached(const void* q, const void* k, const vo
                                           double scale, void* stream_) {
   if (batch < 0 || heads <= 0 || length <= 0 || total < length || dim <= 0 || dim > 256) return QA_EINVAL;
   if ((dtype != BF16 && dtype != F32) || dim % (dtype == F32 ? 4 : 8)) return QA_EINVAL;
-  if (total > CACHED_KEYS || heads > 65536 || batch > 0x7fffffff / heads / length || !(scale > 0.0) || scale > 1e30)
+  // a launch holds fewer than 2^32 threads: 2^22 workgroups of 16 waves are too many
+  if (total > CACHED_KEYS || heads > 65536 || batch > 0x3fffff / heads / length || !(scale > 0.0) || scale > 1e30)
     return QA_EINVAL;
   if (batch == 0) return QA_OK;
   if (!aligned16({q, k, v, out})) return QA_EINVAL;
@@ -237,9 +238,10 @@ extern "C" int qutai_amd_cache_join(const void* past_k, const void* past_v, cons
   if (past_bytes > (1ll << 34) || new_bytes > (1ll << 34)) return QA_EINVAL;  // a row's chunks stay below 2^31
   const int64_t chunks = (past_bytes + new_bytes) / 16, segments = (chunks + JOIN_THREADS * JOIN_DEEP - 1) / (JOIN_THREADS * JOIN_DEEP);
   if (rows == 0 || chunks == 0) return QA_OK;
-  if (rows > 0x7fffffff / 2 / segments) return QA_EINVAL;
-  if ((past_bytes && (!past_k || !past_v)) || (new_bytes && (!new_k || !new_v)) || !out_k || !out_v) return QA_EINVAL;
-  if (!aligned16({past_k, past_v, new_k, new_v, out_k, out_v})) return QA_EINVAL;
+  if (rows > 0x7fffff / segments) return QA_EINVAL;  // 2 x rows x segments workgroups of 256 threads, below 2^32 threads
+  if ((past_bytes && !aligned16({past_k, past_v})) || (new_bytes && !aligned16({new_k, new_v})) ||
+      !aligned16({out_k, out_v}))
+    return QA_EINVAL;
   const JoinArgs a = {{(const u32x4*)past_k, (const u32x4*)past_v}, {(const u32x4*)new_k, (const u32x4*)new_v},
                       {(u32x4*)out_k, (u32x4*)out_v}, (uint32_t)rows, (uint32_t)segments,
                       (uint32_t)(past_bytes / 16), (uint32_t)(new_bytes / 16)};

@@ -33,6 +33,17 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
 
 
+@pytest.mark.skipif(not LIBRARY.exists(), reason="libqutai_amd.so not built")
+def test_launches_of_too_many_threads_are_refused():
+    """2^32 threads or more in one launch: refused before it (no device here)."""
+    from qutai_amd.backends import amd_runtime
+
+    library, p = amd_runtime.load_library(), 4096
+    assert library.qutai_amd_attention_cached(p, p, p, p, 1 << 12, 1 << 10, 1, 1, 8, 5, 1.0, None) == amd_runtime.QA_EINVAL
+    assert library.qutai_amd_cache_join(p, p, p, p, p, p, 1 << 23, 16, 16, None) == amd_runtime.QA_EINVAL
+    assert library.qutai_amd_cache_join(p, p, p, p, p, p, 1 << 22, 1 << 14, 16, None) == amd_runtime.QA_EINVAL
+
+
 def test_python_binding_table_matches_the_header():
     from qutai_amd.backends import amd_runtime
 

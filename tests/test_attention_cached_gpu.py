@@ -70,11 +70,11 @@ def test_cached_attention_refuses_what_its_kernel_cannot_hold():
 
 
 @pytest.mark.parametrize("dtype,batch,heads,past,new,dim", [
-    ("bfloat16", 1, 1, 1, 1, 8), ("float32", 3, 5, 7, 2, 12), ("bfloat16", 2, 3, 127, 1, 64),
+    ("bfloat16", 1, 1, 1, 1, 8), ("bfloat16", 2, 3, 0, 2, 8), ("float32", 1, 2, 0, 1, 64), ("float32", 3, 5, 7, 2, 12), ("bfloat16", 2, 3, 127, 1, 64),
     ("float32", 2, 2, 1023, 2, 4), ("bfloat16", 2, 2, 300, 70, 128), ("float32", 1, 3, 5, 2, 6), ("bfloat16", 1, 2, 3, 1, 20),
 ])
 def test_cache_update_joins_keys_and_values(dtype, batch, heads, past, new, dim):
-    """Rows of one chunk, around one and two segments of 1024 chunks, new positions
+    """An empty cache of its shape, rows of one chunk, around one and two segments of 1024 chunks, new positions
     longer than a workgroup's stride; the last two take the copies."""
     rng = np.random.default_rng(past)
     old, fresh = ([_draw(rng, (batch, heads, n, dim), dtype) for _ in range(2)] for n in (past, new))

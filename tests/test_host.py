@@ -216,6 +216,24 @@ def test_importing_the_package_does_not_touch_the_gpu():
     assert out.returncode == 0 and "lazy" in out.stdout
 
 
+def test_calls_beyond_one_launch_go_elsewhere():
+    """Fewer than 2^32 threads fit a launch: 2^22 queries with a workgroup of
+    1024 each, or 2^23 16 KiB segments of a cache, take the other path."""
+    from types import SimpleNamespace as Store
+
+    from qutai_amd.backends import amd_lm
+
+    def store(size):
+        return Store(dtype="bfloat16", size=size, ptr=4096)
+
+    small = store(1 << 30)
+    for queries, fits in (((1 << 22) - 1, True), (1 << 22, False)):
+        assert amd_lm.attention_cached_serves(store(queries * 8), small, small, 1, 5, 8) is fits
+    for rows, positions in ((1 << 23, 1), (1 << 22, 2048 + 1)):
+        past, new = store(rows * (positions - 1) * 8), store(rows * 8)
+        assert amd_lm.cache_join((past, past), (new, new), rows) is None
+
+
 def test_owned_gradient_marks_are_taken_once():
     """A rule's freshly allocated gradient (grad.owned) is kept by the first
     leaf that receives it; any later receiver copies (core/grad.py)."""
