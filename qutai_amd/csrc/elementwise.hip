@@ -4,6 +4,7 @@
 // All HBM-bound; every kernel moves 16 bytes per lane where the layout
 // allows it.  Reference counterparts are cited per entry point in
 // include/qutai_amd.h.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -249,11 +250,46 @@ __global__ void __launch_bounds__(THREADS) row_partials_kernel(const typename Ac
   }
 }
 
-// inner > 1: a workgroup sums `span` rows of 64 V neighbouring columns (V
+// inner > 1, one lane per (o, part, j) column segment, consecutive lanes on
+// consecutive j; parts == 1 writes the rounded sum, otherwise the fp partials
+// [o][part][j] go to `partial`.  For few inner elements or short sums, where a
+// workgroup's lanes would stand idle (see lane_columns).
+template <class T>
+__global__ void __launch_bounds__(THREADS) col_sum_lanes(const T* __restrict__ x, T* __restrict__ out,
+                                                         typename Acc<T>::R* __restrict__ partial, int64_t outer,
+                                                         int64_t width, int64_t inner, int64_t parts, int64_t span) {
+  typedef typename Acc<T>::R R;
+  const int64_t total = outer * parts * inner;
+  for (int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x; i < total; i += (int64_t)gridDim.x * THREADS) {
+    const int64_t j = i % inner, op = i / inner, part = op % parts, o = op / parts;
+    const int64_t lo = part * span, hi = lo + span < width ? lo + span : width;
+    const T* p = x + o * width * inner + j;
+    R s = R(0);
+    for (int64_t c = lo; c < hi; c++) s += widen(p[c * inner]);
+    if (parts == 1) out[o * inner + j] = narrow<T>(s);
+    else partial[i] = s;
+  }
+}
+
+// The partials of each column in part order, one lane per column.
+template <class T>
+__global__ void __launch_bounds__(THREADS) col_partials_lanes(const typename Acc<T>::R* __restrict__ partial,
+                                                              T* __restrict__ out, int64_t outer, int64_t inner,
+                                                              int64_t parts) {
+  typedef typename Acc<T>::R R;
+  const int64_t total = outer * inner;
+  for (int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x; i < total; i += (int64_t)gridDim.x * THREADS) {
+    const int64_t o = i / inner, j = i % inner;
+    R s = R(0);
+    for (int64_t q = 0; q < parts; q++) s += partial[(o * parts + q) * inner + j];
+    out[i] = narrow<T>(s);
+  }
+}
+
+// The same with a workgroup for `span` rows of 64 V neighbouring columns (V
 // elements, 16 bytes, per lane where rows allow it, else one); its four waves
 // take every fourth row with eight rows' loads in flight, and their sums are
-// added in wave order.  parts == 1 writes the rounded sum, otherwise the fp
-// partials [o][part][j] go to `partial`.  Bound by HBM: 2048 x 3584 fp32 with
+// added in wave order.  Bound by HBM: 2048 x 3584 fp32 with
 // col_partials 40 -> 12 us, 4096 x 512 fp32 34 -> 9 (one row's load at a
 // time per lane, and the partials added by one lane per column, before).
 template <class T, int V>
@@ -404,13 +440,31 @@ void row_plan(int64_t rows, int64_t width, int64_t& parts, int64_t& span) {
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;
 }
-// Column form: about 65536 column segments of at least 64 rows, 256 to a
-// workgroup of the fp32 kernel.
+// Column form: about 65536 column segments of at least 64 rows.
 void col_plan(int64_t columns, int64_t width, int64_t& parts, int64_t& span) {
   parts = reduce_parts(columns, width, 65536, 64);
   span = (width + parts - 1) / parts;
   parts = span ? (width + span - 1) / span : 1;
   if (parts < 1) parts = 1;
+}
+
+// Whether `items` column sums of `span` terms over `inner` columns take a lane
+// each rather than a workgroup per 64 v columns (v elements per lane): the
+// costs in ns of both, fitted to 500 shapes (inner 2 to 1024, 2 to 16384 terms,
+// 2^18 to 2^26 elements, fp32 and bf16).  The GPU starts and ends a workgroup
+// every 0.8 to 1.5 ns and goes through its rows at the second term, however few
+// of its lanes have a column; all of them read at most 950 v elements a ns.  A
+// lane waits 400 ns for each term, less where neighbouring rows share a cache
+// line, with 2048 lanes on each of 256 CUs.
+// Within 10% of the faster form on 95% of them; lanes and workgroups, fp32,
+// outer x terms x inner: 8388608 x 2 x 4 124 and 7929 us, 1048576 x 16 x 4 82
+// and 1339, 1024 x 256 x 256 93 and 39.
+bool lane_columns(int64_t items, int64_t span, int64_t inner, int v, int bytes) {
+  const double groups = (double)items * (double)((inner + 64 * v - 1) / (64 * v));
+  const double line = std::min(1.0, std::max(0.4, (double)inner * bytes / 128));
+  const double columns = (double)items * (double)inner, terms = (double)span;
+  return std::max(groups * (0.7 + 0.1 * v + (0.008 + 0.004 * v) * terms), columns * terms / (950.0 * v)) >
+         terms * 400.0 * line * std::max(1.0, columns / 524288);
 }
 
 }  // namespace
@@ -543,13 +597,19 @@ int qutai_amd_reduce_sum(const void* x, void* out, int64_t outer, int64_t width,
     } else {
       col_plan(outer * inner, width, parts, span);
       constexpr int V = Lanes<T>::V;
-      if (inner % V == 0 && (uintptr_t)x % 16 == 0)
+      const bool wide = inner % V == 0 && (uintptr_t)x % 16 == 0;
+      if (lane_columns(outer * parts, span, inner, wide ? V : 1, sizeof(T)))
+        col_sum_lanes<T><<<blocks_for(outer * parts * inner), THREADS, 0, st>>>((const T*)x, (T*)out, partial, outer,
+                                                                                width, inner, parts, span);
+      else if (wide)
         col_sum_kernel<T, V><<<blocks_for(outer * parts * ((inner + 64 * V - 1) / (64 * V)), 1), THREADS, 0, st>>>(
             (const T*)x, (T*)out, partial, outer, width, inner, parts, span);
       else
         col_sum_kernel<T, 1><<<blocks_for(outer * parts * ((inner + 63) / 64), 1), THREADS, 0, st>>>(
             (const T*)x, (T*)out, partial, outer, width, inner, parts, span);
-      if (parts > 1)
+      if (parts > 1 && lane_columns(outer, parts, inner, 1, sizeof(R)))
+        col_partials_lanes<T><<<blocks_for(outer * inner), THREADS, 0, st>>>(partial, (T*)out, outer, inner, parts);
+      else if (parts > 1)
         col_partials_kernel<T><<<blocks_for(outer * ((inner + 63) / 64), 1), THREADS, 0, st>>>(partial, (T*)out, outer,
                                                                                              inner, parts);
     }

@@ -32,6 +32,18 @@ def test_column_sums(amd, dtype, outer, rows, cols):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float64"])
+@pytest.mark.parametrize("outer,rows,cols", [(20001, 16, 4), (20001, 2, 3), (20000, 130, 2), (2000, 17, 16), (3, 300, 2),
+                                             (1, 20000, 2), (4000, 64, 8), (500, 5, 100)])
+def test_column_sums_of_few_columns(amd, dtype, outer, rows, cols):
+    """A lane per column, with one and two parts, and shapes on both sides of
+    the line to a workgroup per column block.  Chains of at most 65 terms."""
+    x = normal(rows * cols, outer * rows * cols)
+    got = download(amd.sum(upload(x, dtype), (outer, rows, cols), 1)).reshape(outer, cols)
+    exact = stored(x, dtype).reshape(outer, rows, cols).sum(1)
+    assert ora.rel_frobenius(got, exact) <= BAR[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float64"])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (3, 4), (257, 24), (100, 513), (64, 1024)])
 def test_bias_add(amd, dtype, rows, cols):
     x, bias = normal(rows, rows * cols), normal(cols, cols)
