@@ -32,7 +32,12 @@ void launch_pass(Pass pass, const AttnGenArgs& a, unsigned blocks, hipStream_t s
   const dim3 grid(blocks), block(256);
   if (pass == FORWARD) hipLaunchKernelGGL((attention_fwd_mma<F32, DP>), grid, block, 0, stream, a);
   else if (pass == QUERIES) hipLaunchKernelGGL((attention_bwd_dq_mma<F32, DP>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((attention_bwd_dkv_mma<F32, DP>), grid, block, 0, stream, a);
+  else if constexpr (DP > 128) {
+    hipLaunchKernelGGL((attention_bwd_dkv_mma<F32, DP, KEYS_DV>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attention_bwd_dkv_mma<F32, DP, KEYS_DK>), grid, block, 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((attention_bwd_dkv_mma<F32, DP, KEYS_BOTH>), grid, block, 0, stream, a);
+  }
 }
 
 // The kernel width DP is the smallest built one that holds the head

@@ -10,8 +10,7 @@
 //    values takes the six MFMAs whose terms are above 2^-24 of it, so an fp32
 //    product costs 6/16 of v_mfma_f32_32x32x2_f32's cycles;
 //  * fp32 storage splits q, k, v and dO that way, both storage types split the
-//    probabilities and dS: three parts for fp32 storage, two (2^-17) for
-//    bf16 storage, where the result is rounded to bf16;
+//    probabilities and dS, which are fp32 in either;
 //  * the split needs finite values; an infinity or NaN anywhere in a wave's
 //    operands reaches its accumulators as a NaN or infinity, and such a wave
 //    computes its rows again with the one-wave-per-row code.
@@ -26,12 +25,13 @@
 // (the same lane layout as the D = 64 kernels).
 //
 // What bounds it: the MFMAs (fp32: 12 per 32x32 scores and 16 dimensions in
-// the forward, bf16: 3) and the splitting of the probabilities beside them.
-// Measured (MI355X, causal; forward, dq, dk/dv), against one wave per row:
-// bf16, batch 4, T 1024, 16 heads over 4 of 128: 5663, 5315, 8195 us before,
-// 45, 61, 101 (+ 12 for the sum over the heads of a group) now; fp32, batch 8,
-// T 512, 8 heads of 64: 1236, 1433, 1429 us before, 35, 43, 61 now, and the
-// error against float64 is 0.3 to 0.9 of what it was.
+// the forward, bf16: 4) and the splitting of the probabilities beside them.
+// Measured (MI355X, causal; forward and backward), against one wave per row:
+// bf16, batch 4, T 1024, 16 heads over 4 of 128: 5663 and 13510 us before, 58
+// and 222 now; fp32, batch 8, T 512, 8 heads of 64: 1236 and 2862 us before, 34
+// and 98 now.  With two parts (2^-17) of the probabilities and dS the first
+// takes 45 and 168 us, but 2.3 of 1000 bf16 results were not float64's rounded,
+// 0.5 with one wave per row, 0.3 with three parts.
 #pragma once
 #include "attention_rows.h"
 
@@ -71,7 +71,7 @@ using namespace qa;
 template <bool F32, int DP>
 struct AttnTile {
   static constexpr int NX = F32 ? 3 : 1;             // parts of a stored value
-  static constexpr int NP = F32 ? 3 : 2;             // parts of a probability or dS
+  static constexpr int NP = 3;                       // parts of a probability or dS
   static constexpr int KB = F32 || DP > 128 ? 32 : 64;
   static constexpr int CK = DP / 8;                  // chunks of a row in use
   static constexpr int PC = DP <= 32 ? 4 : DP <= 64 ? 8 : DP <= 128 ? 16 : 32;
@@ -215,14 +215,10 @@ __device__ __forceinline__ void add_product(const bf16_t* x, int db, int mb, int
   for (int st = 0; st < 2; st++) {
     bf16x8 f[Tile::NX];
     Tile::columns(x, db, 32 * mb + 16 * st, lane, f);
-    if constexpr (F32) {
-      acc = high_part(f, w[st], acc);
-      lo = mma_parts(f, w[st], lo, 1);
-    } else {
-      acc = mma_parts(f, w[st], acc);
-    }
+    acc = high_part(f, w[st], acc);
+    lo = mma_parts(f, w[st], lo, 1);
   }
-  if constexpr (F32) acc += lo;
+  acc += lo;
 }
 
 // Four consecutive outputs d .. d+3 of one row.
@@ -545,9 +541,14 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
 }
 
 // dK and dV of 128 keys of one kv head (p.split: of one query head of its
-// group, as unscaled fp32 partials); Q, dO, lse and delta stream.
-template <bool F32, int DP>
-__global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 96 ? 1 : 2) attention_bwd_dkv_mma(AttnGenArgs p) {
+// group, as unscaled fp32 partials); Q, dO, lse and delta stream.  Above 128
+// dimensions the sums of both do not fit a wave's registers and each has a
+// launch (bf16, batch 4, T 1024, 16 heads over 4 of 256: a backward pass takes
+// 555 us, 1295 with both and their spills).
+enum KeySide { KEYS_BOTH, KEYS_DK, KEYS_DV };
+
+template <bool F32, int DP, KeySide SIDE>
+__global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 64 ? 1 : 2) attention_bwd_dkv_mma(AttnGenArgs p) {
   typedef AttnTile<F32, DP> Tile;
   typedef AttnStage<F32, DP> Stage;
   typedef typename std::conditional<F32, float, bf16_t>::type T_;
@@ -586,9 +587,12 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 96 ? 1 : 2) attent
 #pragma unroll
     for (int s = 0; s < Tile::S; s++) raw[s].parts(vf[s]);
   }
-  f32x16 dkt[Tile::DB], dvt[Tile::DB];
+  constexpr bool DK = SIDE != KEYS_DV, DV = SIDE != KEYS_DK;
+  f32x16 dkt[DK ? Tile::DB : 1], dvt[DV ? Tile::DB : 1];
 #pragma unroll
-  for (int db = 0; db < Tile::DB; db++) dkt[db] = dvt[db] = f32x16{};
+  for (auto& x : dkt) x = f32x16{};
+#pragma unroll
+  for (auto& x : dvt) x = f32x16{};
 
   const int qs0 = p.causal ? k0 : 0;
   const int nq = qs0 < T ? (T - qs0 + KB - 1) / KB : 0;
@@ -629,16 +633,19 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 96 ? 1 : 2) attent
       Tile::rows(sq, 32 * mb + col, s, half, qa);
       sc = high_part(qa, kf[s], sc);
       if constexpr (F32) sc_lo = mma_parts(qa, kf[s], sc_lo, 1);
-      Tile::rows(sg, 32 * mb + col, s, half, ga);
-      dp = high_part(ga, vf[s], dp);
-      if constexpr (F32) dp_lo = mma_parts(ga, vf[s], dp_lo, 1);
+      if constexpr (DK) {
+        Tile::rows(sg, 32 * mb + col, s, half, ga);
+        dp = high_part(ga, vf[s], dp);
+        if constexpr (F32) dp_lo = mma_parts(ga, vf[s], dp_lo, 1);
+      }
     }
     if constexpr (F32) sc += sc_lo, dp += dp_lo;
     // element e: query qs + 32 mb + 8 (e / 4) + 4 half + e % 4, key kw + col
-    bf16x8 pf[2][Tile::NP], dsf[2][Tile::NP];
+    float ds[16];
+    bf16x8 w[2][Tile::NP];  // the probabilities, then dS
 #pragma unroll
     for (int st = 0; st < 2; st++) {
-      float pr[8], ds[8];
+      float pr[8];
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const int q4 = 32 * mb + 8 * (2 * st + j) + 4 * half;
@@ -653,16 +660,20 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 96 ? 1 : 2) attent
           if constexpr (decltype(mask)::value)
             if (qs + q4 + i >= T || (p.causal && qs + q4 + i < key)) x = -INFINITY;
           pr[4 * j + i] = weight_of<F32>(x, p, l4[i], lo4[i]);
-          ds[4 * j + i] = pr[4 * j + i] * (dp[e] - d4[i]);
+          ds[e] = pr[4 * j + i] * (dp[e] - d4[i]);
         }
       }
-      split_bf16(pr, pf[st]);
-      split_bf16(ds, dsf[st]);
+      if constexpr (DV) split_bf16(pr, w[st]);
     }
+    if constexpr (DV) {
 #pragma unroll
-    for (int db = 0; db < Tile::DB; db++) {
-      add_product<F32, DP>(sg, db, mb, lane, pf, dvt[db]);
-      add_product<F32, DP>(sq, db, mb, lane, dsf, dkt[db]);
+      for (int db = 0; db < Tile::DB; db++) add_product<F32, DP>(sg, db, mb, lane, w, dvt[db]);
+    }
+    if constexpr (DK) {
+#pragma unroll
+      for (int st = 0; st < 2; st++) split_bf16(reinterpret_cast<const float(&)[8]>(ds[8 * st]), w[st]);
+#pragma unroll
+      for (int db = 0; db < Tile::DB; db++) add_product<F32, DP>(sq, db, mb, lane, w, dkt[db]);
     }
   };
   // per head: query blocks before every key of the wave (causal; skipped),
@@ -705,15 +716,18 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 96 ? 1 : 2) attent
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         const int d = 32 * db + 8 * g + 4 * half;
-        const f32x4 xk = {dkt[db][4 * g], dkt[db][4 * g + 1], dkt[db][4 * g + 2], dkt[db][4 * g + 3]};
-        const f32x4 xv = {dvt[db][4 * g], dvt[db][4 * g + 1], dvt[db][4 * g + 2], dvt[db][4 * g + 3]};
         if (d >= D) continue;
-        if (p.split) {
-          global_store(p.part_k + gsel * p.part_stride + at + d, xk);
-          global_store(p.part_v + gsel * p.part_stride + at + d, xv);
-        } else {
-          put4<F32>(p.dk, at + d, xk * p.scale);
-          put4<F32>(p.dv, at + d, xv);
+        if constexpr (DK) {
+          const f32x16& y = dkt[db];
+          const f32x4 x = {y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]};
+          if (p.split) global_store(p.part_k + gsel * p.part_stride + at + d, x);
+          else put4<F32>(p.dk, at + d, x * p.scale);
+        }
+        if constexpr (DV) {
+          const f32x16& y = dvt[db];
+          const f32x4 x = {y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]};
+          if (p.split) global_store(p.part_v + gsel * p.part_stride + at + d, x);
+          else put4<F32>(p.dv, at + d, x);
         }
       }
   }
