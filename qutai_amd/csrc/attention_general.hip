@@ -76,6 +76,20 @@ void set_scale(AttnGenArgs& a, double scale) {
 
 constexpr int64_t OWNED = 128;  // queries or keys of a workgroup
 
+// Whether a call takes one wave per row although the matrix kernels could hold
+// it: the tiles of a sequence of a few positions are mostly empty, and sums of
+// one or two terms round best on their own.  Measured with 16000 heads (us;
+// rows, tiles): forward bf16 D 128, T 6 103 and 178, T 8 191 and 180; bf16 D 32,
+// T 6 72 and 75; fp32 D 64, T 8 128 and 148; backward bf16 D 128 with a quarter of
+// the kv heads, T 2 45 and 723, T 12 618 and 739; bf16 D 32, T 6 153 and 168, T 8
+// 279 and 168; fp32 D 32, T 8 270 and 312.  Grids of fewer heads than the GPU
+// holds at once take the tiles earlier (32 heads of 128, bf16: forward, T 3, 10 and
+// 7.6; backward, T 4, 20 and 22, T 5 24 and 22).
+bool few_positions(int dtype, int64_t batch, int64_t heads, int64_t time, int64_t dim, bool backward) {
+  const int64_t most = dim > 32 ? (backward ? 12 : 8) : backward && dtype == F32 ? 8 : 6;
+  return time <= (backward ? 4 : 2) || (time <= most && batch * heads >= 2 * cu_count());
+}
+
 // Partial dK/dV of the query heads of each kv head's group, for grids of
 // fewer workgroups than the GPU holds at once (two per CU).
 size_t split_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim) {
@@ -103,7 +117,7 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
   a.causal = causal ? 1 : 0;
   const int64_t rows = batch * heads * time;
   if ((rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
-  if (mma_fits(dtype, dim) && aligned16({q, k, v, out}))
+  if (mma_fits(dtype, dim) && aligned16({q, k, v, out}) && !few_positions(dtype, batch, heads, time, dim, false))
     return (int)launch_mma(FORWARD, dtype, a, batch * heads * ((time + OWNED - 1) / OWNED), stream);
   return (int)launch_rows(attention_fwd_rows<bf16_t>, attention_fwd_rows<float>, dtype, a, rows, stream);
 }
@@ -111,6 +125,7 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
 size_t attention_general_workspace(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim,
                                    int dtype) {
   if ((dtype != BF16 && dtype != F32) || dim <= 0 || batch < 0 || time < 0 || !mma_fits(dtype, dim)) return 0;
+  if (few_positions(dtype, batch, heads, time, dim, true)) return 0;
   return split_bytes(batch, heads, kv_heads, time, dim);
 }
 
@@ -138,7 +153,8 @@ int attention_general_bwd(const void* grad, const void* q, const void* k, const 
   const int64_t q_rows = batch * heads * time, k_rows = batch * kv_heads * time;
   if ((q_rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
   // the q pass writes delta, which the kv pass reads
-  if (!mma_fits(dtype, dim) || !aligned16({grad, q, k, v, out, dq, dk, dv})) {
+  if (!mma_fits(dtype, dim) || !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
+      few_positions(dtype, batch, heads, time, dim, true)) {
     const hipError_t e =
         launch_rows(attention_bwd_q_rows<bf16_t>, attention_bwd_q_rows<float>, dtype, a, q_rows, stream);
     if (e != hipSuccess) return (int)e;

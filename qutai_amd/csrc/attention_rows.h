@@ -5,8 +5,9 @@
 // query row (forward, dq) or key row (dk, dv); lane l owns dimensions l,
 // l + 64, l + 128, l + 192; dot products are wave-wide sums.  Bound by the
 // cross-lane sums of every score, so it serves the rows that the matrix
-// kernels (attention_mma.h) leave: rows that are not 16-byte aligned, and
-// waves whose operands hold an infinity or a NaN.
+// kernels (attention_mma.h) leave: rows that are not 16-byte aligned,
+// sequences of a few positions, and waves whose operands hold an infinity or
+// a NaN.
 #pragma once
 #include "attention_common.h"
 

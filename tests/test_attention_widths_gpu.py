@@ -117,3 +117,32 @@ def test_a_query_of_one_key_has_no_gradient(lm, dims):
     and dQ is an exact zero (as float64 has it), not what two roundings leave."""
     _, (out, dq, _, _), _ = run(lm, "bfloat16", dims, True, 1)
     assert not dq[:, :, 0].any() and out[:, :, 0].any()
+
+
+@pytest.mark.parametrize("dtype,dim", [("bfloat16", 32), ("bfloat16", 128), ("float32", 32), ("float32", 64)])
+@pytest.mark.parametrize("time", [1, 2, 3, 6, 7, 8, 9, 12, 13])
+@pytest.mark.parametrize("heads", [2, 512])
+def test_short_sequences(lm, dtype, dim, time, heads):
+    """Both sides of the lines between one wave per row and tiles, for grids that
+    fill the GPU and that do not."""
+    (q, k, v, g), (out, dq, dk, dv), _ = run(lm, dtype, (1, time, heads, heads, dim), True, 1)
+    for h in (0, heads - 1):
+        o_ref, l_ref = ora.attention_np(q[0, h], k[0, h], v[0, h])
+        grads = ora.attention_backward_np(g[0, h], q[0, h], k[0, h], v[0, h], out[0, h], l_ref)
+        assert ora.rel_frobenius(out[0, h], o_ref) <= BAR[dtype]
+        for got, exact in zip((dq, dk, dv), grads):
+            # dq and dk of one position are a difference of equal sums
+            assert np.linalg.norm(got[0, h] - exact) <= BAR[dtype] * max(np.linalg.norm(exact), np.linalg.norm(grads[2]))
+
+
+def test_more_short_sequences_than_a_launch_holds_tiles(lm):
+    """2^24 heads of one position: as many tiles of 256 threads are 2^32 threads,
+    which no launch holds.  Each output is its value."""
+    from qutai_amd.backends import amd
+
+    batch, heads, dim = 4096, 4096, 8
+    one, two = (amd.full(batch * heads * dim, x, dtype="bfloat16") for x in (1.0, 2.0))
+    out, lse = lm.attention(one, one, two, batch, 1, heads, heads, dim)
+    dq, dk, dv = lm.attention_backward(one, one, one, two, out, lse, batch, 1, heads, heads, dim)
+    for got, value in ((out, 2.0), (dq, 0.0), (dk, 0.0), (dv, 1.0)):
+        assert (np.frombuffer(got.to_array(), np.uint16) == np.float32(value).view(np.uint32) >> 16).all()
