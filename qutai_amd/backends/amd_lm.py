@@ -483,6 +483,20 @@ def attention_cached_serves(q, k, v, length, total, dim):
             and all(x.ptr % 16 == 0 for x in (q, k, v)))
 
 
+def attention_cached_gains(q, length, total, dim):
+    """Whether ``attention_cached`` is faster than the products for operands that
+    it takes: for one query, and for fp32, throughout.  Several bf16 queries, in
+    ns for each (batch, head): a workgroup costs 8.6 and 0.03 a key of 64, the
+    products 10 + 15 and 0.36, and 100 us more of host time (2000 batches, 8 heads
+    of 64, a layer call of 8 queries over 8 keys 1582 us and 891 with the products,
+    8 over 135 2246 and 1704, 4 over 35 1046 and 1038, 4 over 131 1456 and 1518)."""
+    if length == 1 or q.dtype != "bfloat16":
+        return True
+    pairs, wide = q.size // (length * dim), dim / 64
+    queries, products = length * (8.6 + 0.03 * wide * total), 10 + 15 * wide + 0.36 * wide * total
+    return pairs * (queries - products) <= 100_000
+
+
 def attention_cached(q, k, v, batch, length, total, heads, dim):
     """softmax(Q K^T / sqrt(dim)) V of ``length`` new positions over the
     (batch, heads, total, dim) cache that ends with them; q and the result are

@@ -174,7 +174,8 @@ class MultiHeadAttention(Attention):
             batch, length, features = tensor.shape
             total, dim = keys.shape[2:]
             stores = tuple(x.storage for x in (queries, keys, values))
-            if matmul_precision() is None and amd_lm.attention_cached_serves(*stores, length, total, dim):
+            if (matmul_precision() is None and amd_lm.attention_cached_serves(*stores, length, total, dim)
+                    and amd_lm.attention_cached_gains(stores[0], length, total, dim)):
                 mixed = amd_lm.attention_cached(*stores, batch, length, total, self.heads, dim)
                 return self.output(Tensor(mixed, shape=(batch, length, features)))
             scores = matmul(self._split(queries), keys.transpose((0, 1, 3, 2)))

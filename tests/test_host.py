@@ -234,6 +234,20 @@ def test_calls_beyond_one_launch_go_elsewhere():
         assert amd_lm.cache_join((past, past), (new, new), rows) is None
 
 
+def test_many_short_cached_queries_take_the_products():
+    from types import SimpleNamespace as Store
+
+    from qutai_amd.backends.amd_lm import attention_cached_gains
+
+    def gains(dtype, pairs, length, total, dim):
+        return attention_cached_gains(Store(dtype=dtype, size=pairs * length * dim), length, total, dim)
+
+    assert gains("bfloat16", 16000, 1, 8, 64) and gains("float32", 16000, 8, 8, 64)
+    assert gains("bfloat16", 512, 8, 8, 64) and gains("bfloat16", 512, 8, 4000, 128)
+    assert not gains("bfloat16", 16000, 8, 8, 64) and not gains("bfloat16", 16000, 8, 135, 64)
+    assert not gains("bfloat16", 16000, 4, 8, 64) and gains("bfloat16", 16000, 4, 131, 64)
+
+
 def test_owned_gradient_marks_are_taken_once():
     """A rule's freshly allocated gradient (grad.owned) is kept by the first
     leaf that receives it; any later receiver copies (core/grad.py)."""
