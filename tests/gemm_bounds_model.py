@@ -120,11 +120,13 @@ def records(nbytes: int, clamped: bool = True) -> int:
 
 
 def part_stages(cfg: Config, k_len: int) -> list[int]:
-    """First k of every stage (16 of K) that reduce_parts fetches: one stage
-    ahead on 256x256 tiles, which skip stages past the next; two on smaller
-    ones, whose steps come in pairs and fetch without a condition."""
+    """First k of every stage (16 of K) that reduce_parts fetches: the only one
+    (but on the 256x64 tile); else one stage ahead on 256x256 tiles, which skip stages past the next; two
+    on smaller ones, whose steps come in pairs and fetch without a condition."""
     depth = 1 if cfg.bm * cfg.bn >= 256 * 256 else 2
     nk = (k_len + 15) // 16
+    if nk <= 1 and (cfg.bm, cfg.bn) != (256, 64):
+        return [0]
     steps = [kt for kt in range(nk) if kt + 1 < nk] if depth == 1 else range(nk + nk % 2)
     return [16 * s for s in sorted({*range(depth + 1), *(kt + 1 + depth for kt in steps)})]
 
