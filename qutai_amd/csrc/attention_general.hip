@@ -45,6 +45,10 @@ void launch_pass(Pass pass, const AttnGenArgs& a, unsigned blocks, hipStream_t s
 // need more registers than a wave has (three parts of q and dO).
 bool mma_fits(int dtype, int64_t dim) { return dtype == BF16 ? dim % 8 == 0 && dim <= 256 : dim % 4 == 0 && dim <= 128; }
 
+// A scale of the scores with which the factors that take the parts' scaling
+// back (2^-48 at most) keep their bits: any in earnest use.
+bool mma_scale(double scale) { return scale >= 0x1p-50; }
+
 hipError_t launch_mma(Pass pass, int dtype, const AttnGenArgs& a, int64_t blocks, hipStream_t stream) {
   const unsigned n = (unsigned)blocks;
   if (dtype == BF16) {
@@ -68,10 +72,13 @@ hipError_t launch_rows(Kernel bf16, Kernel fp32, int dtype, const AttnGenArgs& a
   return hipGetLastError();
 }
 
-void set_scale(AttnGenArgs& a, double scale) {
+// scale_log2 takes the scores of the matrix kernels, products of two stored
+// values as they are scaled (AttnTile::STORED)
+void set_scale(AttnGenArgs& a, double scale, int dtype) {
   a.scale = (float)scale;
-  a.scale_log2 = (float)(scale * 1.4426950408889634);
-  a.scale_log2_lo = (float)(scale * 1.4426950408889634 - (double)a.scale_log2);
+  const double log2 = scale * 1.4426950408889634 * (dtype == F32 ? 0x1p-48 : 1.0);
+  a.scale_log2 = (float)log2;
+  a.scale_log2_lo = (float)(log2 - (double)a.scale_log2);
 }
 
 constexpr int64_t OWNED = 128;  // queries or keys of a workgroup
@@ -113,11 +120,12 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
   a.dq = out;
   a.lse = lse;
   a.dim = dim;
-  set_scale(a, scale);
+  set_scale(a, scale, dtype);
   a.causal = causal ? 1 : 0;
   const int64_t rows = batch * heads * time;
   if ((rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
-  if (mma_fits(dtype, dim) && aligned16({q, k, v, out}) && !few_positions(dtype, batch, heads, time, dim, false))
+  if (mma_fits(dtype, dim) && mma_scale(scale) && aligned16({q, k, v, out}) &&
+      !few_positions(dtype, batch, heads, time, dim, false))
     return (int)launch_mma(FORWARD, dtype, a, batch * heads * ((time + OWNED - 1) / OWNED), stream);
   return (int)launch_rows(attention_fwd_rows<bf16_t>, attention_fwd_rows<float>, dtype, a, rows, stream);
 }
@@ -148,12 +156,12 @@ int attention_general_bwd(const void* grad, const void* q, const void* k, const 
   a.dk = dk;
   a.dv = dv;
   a.dim = dim;
-  set_scale(a, scale);
+  set_scale(a, scale, dtype);
   a.causal = causal ? 1 : 0;
   const int64_t q_rows = batch * heads * time, k_rows = batch * kv_heads * time;
   if ((q_rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
   // the q pass writes delta, which the kv pass reads
-  if (!mma_fits(dtype, dim) || !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
+  if (!mma_fits(dtype, dim) || !mma_scale(scale) || !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
       few_positions(dtype, batch, heads, time, dim, true)) {
     const hipError_t e =
         launch_rows(attention_bwd_q_rows<bf16_t>, attention_bwd_q_rows<float>, dtype, a, q_rows, stream);

@@ -11,9 +11,13 @@
 //    product costs 6/16 of v_mfma_f32_32x32x2_f32's cycles;
 //  * fp32 storage splits q, k, v and dO that way, both storage types split the
 //    probabilities and dS, which are fp32 in either;
-//  * the split needs finite values; an infinity or NaN anywhere in a wave's
-//    operands reaches its accumulators as a NaN or infinity, and such a wave
-//    computes its rows again with the one-wave-per-row code.
+//  * values, probabilities and dS are split as 2^24 of themselves, and the
+//    scale and the outputs' factors take that back: the bits of every finite
+//    value, subnormals included, then end above bf16's smallest normal;
+//  * the split needs finite values, and sums below 2^128 as scaled; an
+//    infinity or NaN anywhere in a wave's operands reaches its accumulators as
+//    a NaN or infinity, and such a wave computes its rows again with the
+//    one-wave-per-row code.
 //
 // Shape of the work: a workgroup of four waves owns 128 queries (forward,
 // dq) or 128 keys (dk, dv) of one (batch, head), 32 per wave; the other
@@ -27,9 +31,9 @@
 // What bounds it: the MFMAs (fp32: 12 per 32x32 scores and 16 dimensions in
 // the forward, bf16: 4) and the splitting of the probabilities beside them.
 // Measured (MI355X, causal; forward and backward), against one wave per row:
-// bf16, batch 4, T 1024, 16 heads over 4 of 128: 5663 and 13510 us before, 58
-// and 222 now; fp32, batch 8, T 512, 8 heads of 64: 1236 and 2862 us before, 34
-// and 98 now.  With two parts (2^-17) of the probabilities and dS the first
+// bf16, batch 4, T 1024, 16 heads over 4 of 128: 5663 and 13510 us before, 60
+// and 227 now; fp32, batch 8, T 512, 8 heads of 64: 1236 and 2862 us before, 35
+// and 102 now.  With two parts (2^-17) of the probabilities and dS the first
 // takes 45 and 168 us, but 2.3 of 1000 bf16 results were not float64's rounded,
 // 0.5 with one wave per row, 0.3 with three parts.
 #pragma once
@@ -73,6 +77,11 @@ template <bool F32, int DP>
 struct AttnTile {
   static constexpr int NX = F32 ? 3 : 1;             // parts of a stored value
   static constexpr int NP = 3;                       // parts of a probability or dS
+  // what parts of stored values and of probabilities and dS are scaled by,
+  // what takes a sum of products of a stored value and a weight back, and dP
+  // (two stored values) to dS's scale
+  static constexpr float STORED = F32 ? 0x1p24f : 1.f, WEIGHT = 0x1p24f;
+  static constexpr float SUM = 1.f / (STORED * WEIGHT), DP_TO_DS = WEIGHT / (STORED * STORED);
   static constexpr int KB = F32 || DP > 128 ? 32 : 64;
   static constexpr int CK = DP / 8;                  // chunks of a row in use
   static constexpr int PC = DP <= 32 ? 4 : DP <= 64 ? 8 : DP <= 128 ? 16 : 32;
@@ -125,17 +134,11 @@ struct Raw8 {
     if constexpr (F32)
       w[1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, ok_hi ? off + 16 : ATTN_OOB, 0, 0));
   }
-  __device__ __forceinline__ void values(float (&v)[8]) const {
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      if constexpr (F32) v[e] = __uint_as_float(w[e >> 2][e & 3]);
-      else v[e] = __uint_as_float((e & 1) ? (w[0][e >> 1] & 0xffff0000u) : (w[0][e >> 1] << 16));
-    }
-  }
   __device__ __forceinline__ void parts(bf16x8 (&f)[F32 ? 3 : 1]) const {
     if constexpr (F32) {
       float v[8];
-      values(v);
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[e] = __uint_as_float(w[e >> 2][e & 3]) * 0x1p24f;  // AttnTile::STORED
       split_bf16(v, f);
     } else {
       f[0] = __builtin_bit_cast(bf16x8, w[0]);
@@ -361,6 +364,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
       for (int e = 0; e < 8; e++) {
         pv[e] = weight_of<F32>(sc[8 * st + e], p, ref, 0.f);
         sum += pv[e];
+        pv[e] *= Tile::WEIGHT;
       }
       split_bf16(pv, pf[st]);
     }
@@ -391,7 +395,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
     return;
   }
   if (t < T) {
-    const float inv = 1.f / total;
+    const float inv = Tile::SUM / total;
     const int64_t at = b * p.qb + h * p.qh + (int64_t)t * p.qt;
 #pragma unroll
     for (int db = 0; db < Tile::DB; db++)
@@ -463,7 +467,8 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
     dl = pair_sum(dl);
     const int64_t li = b * p.lb + h * p.lh + (int64_t)t * p.lt;
     if (t < T) lse2 = log2_of(p.lse[li], lse2_lo);
-    if (t < T && half == 0) p.delta[li] = dl;
+    if (t < T && half == 0) p.delta[li] = dl * (1.f / (Tile::STORED * Tile::STORED));
+    dl *= Tile::DP_TO_DS;
   }
   f32x16 dqt[Tile::DB];
 #pragma unroll
@@ -509,7 +514,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
         float x = sc[e];
         if constexpr (decltype(mask)::value)
           if (32 * mb + 8 * (e >> 2) + (e & 3) >= lim) x = -INFINITY;
-        ds[i] = weight_of<F32>(x, p, lse2, lse2_lo) * (dp[e] - dl);
+        ds[i] = weight_of<F32>(x, p, lse2, lse2_lo) * __builtin_fmaf(dp[e], Tile::DP_TO_DS, -dl);
       }
       split_bf16(ds, dsf[st]);
     }
@@ -545,7 +550,8 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
         const int d = 32 * db + 8 * g + 4 * half;
         if (d < D)
           put4<F32>(p.dq, at + d,
-                    f32x4{dqt[db][4 * g], dqt[db][4 * g + 1], dqt[db][4 * g + 2], dqt[db][4 * g + 3]} * p.scale);
+                    f32x4{dqt[db][4 * g], dqt[db][4 * g + 1], dqt[db][4 * g + 2], dqt[db][4 * g + 3]} *
+                        (p.scale * Tile::SUM));
       }
   }
 }
@@ -554,7 +560,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 64 || DP > 128 ? 1 : 2) atten
 // group, as unscaled fp32 partials); Q, dO, lse and delta stream.  Above 128
 // dimensions the sums of both do not fit a wave's registers and each has a
 // launch (bf16, batch 4, T 1024, 16 heads over 4 of 256: a backward pass takes
-// 555 us, 1295 with both and their spills).
+// 637 us, about twice that with both and their spills).
 enum KeySide { KEYS_BOTH, KEYS_DK, KEYS_DV };
 
 template <bool F32, int DP, KeySide SIDE>
@@ -564,7 +570,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 64 ? 1 : 2) attent
   typedef typename std::conditional<F32, float, bf16_t>::type T_;
   constexpr int KB = Tile::KB, KPB = 128, ES = F32 ? 4 : 2;
   __shared__ __attribute__((aligned(16))) bf16_t tiles[2 * Tile::NX * Tile::PLANE];  // [Q, dO][plane]
-  __shared__ __attribute__((aligned(16))) float stats[3][KB];  // lse log2(e) and its rounding error, delta
+  __shared__ __attribute__((aligned(16))) float stats[3][KB];  // lse log2(e) and its rounding error, delta as dS
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform32(tid >> 6), half = lane >> 5, col = lane & 31;
   const int T = (int)p.time, D = (int)p.dim;
   const int blocks_k = (T + KPB - 1) / KPB;
@@ -628,7 +634,7 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 64 ? 1 : 2) attent
       float lo;
       stats[0][tid] = log2_of(lse_next, lo);
       stats[1][tid] = lo;
-      stats[2][tid] = delta_next;
+      stats[2][tid] = delta_next * Tile::WEIGHT;
     }
     __syncthreads();
     if (it + 1 < iterations) fetch(it + 1);
@@ -670,7 +676,8 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 64 ? 1 : 2) attent
           if constexpr (decltype(mask)::value)
             if (qs + q4 + i >= T || (p.causal && qs + q4 + i < key)) x = -INFINITY;
           pr[4 * j + i] = weight_of<F32>(x, p, l4[i], lo4[i]);
-          ds[e] = pr[4 * j + i] * (dp[e] - d4[i]);
+          ds[e] = pr[4 * j + i] * __builtin_fmaf(dp[e], Tile::DP_TO_DS, -d4[i]);
+          pr[4 * j + i] *= Tile::WEIGHT;
         }
       }
       if constexpr (DV) split_bf16(pr, w[st]);
@@ -730,14 +737,14 @@ __global__ void __launch_bounds__(256, F32 && DP > 32 || DP > 64 ? 1 : 2) attent
         if constexpr (DK) {
           const f32x16& y = dkt[db];
           const f32x4 x = {y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]};
-          if (p.split) global_store(p.part_k + gsel * p.part_stride + at + d, x);
-          else put4<F32>(p.dk, at + d, x * p.scale);
+          if (p.split) global_store(p.part_k + gsel * p.part_stride + at + d, x * Tile::SUM);
+          else put4<F32>(p.dk, at + d, x * (p.scale * Tile::SUM));
         }
         if constexpr (DV) {
           const f32x16& y = dvt[db];
           const f32x4 x = {y[4 * g], y[4 * g + 1], y[4 * g + 2], y[4 * g + 3]};
-          if (p.split) global_store(p.part_v + gsel * p.part_stride + at + d, x);
-          else put4<F32>(p.dv, at + d, x);
+          if (p.split) global_store(p.part_v + gsel * p.part_stride + at + d, x * Tile::SUM);
+          else put4<F32>(p.dv, at + d, x * Tile::SUM);
         }
       }
   }

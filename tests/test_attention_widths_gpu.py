@@ -25,7 +25,7 @@ def lm():
     return amd_lm
 
 
-def run(lm, dtype, dims, causal, layout, change=None):
+def run(lm, dtype, dims, causal, layout, change=None, scale=None):
     """Device results and stored inputs as [batch][heads][time][dim] float64."""
     batch, time, heads, kv_heads, dim = dims
     counts = (heads, kv_heads, kv_heads, heads)
@@ -39,8 +39,8 @@ def run(lm, dtype, dims, causal, layout, change=None):
     if change:
         change(*(split(x, n) for x, n in zip(host, counts)))
     q, k, v, g = (upload(x, dtype) for x in host)
-    out, lse = lm.attention(q, k, v, *dims, causal=causal, layout=layout)
-    grads = lm.attention_backward(g, q, k, v, out, lse, *dims, causal=causal, layout=layout)
+    out, lse = lm.attention(q, k, v, *dims, causal=causal, layout=layout, scale=scale)
+    grads = lm.attention_backward(g, q, k, v, out, lse, *dims, causal=causal, layout=layout, scale=scale)
     inputs = [split(stored(x, dtype), n) for x, n in zip(host, counts)]
     results = [split(download(x).astype(np.float64), n) for x, n in zip((out, *grads), (heads, heads, kv_heads, kv_heads))]
     lse = download(lse).reshape((batch, time, heads) if layout else (batch, heads, time))
@@ -146,3 +146,26 @@ def test_more_short_sequences_than_a_launch_holds_tiles(lm):
     dq, dk, dv = lm.attention_backward(one, one, one, two, out, lse, batch, 1, heads, heads, dim)
     for got, value in ((out, 2.0), (dq, 0.0), (dk, 0.0), (dv, 1.0)):
         assert (np.frombuffer(got.to_array(), np.uint16) == np.float32(value).view(np.uint32) >> 16).all()
+
+
+# Small magnitudes of q, k, v and dO: all bits count.  Results that are
+# subnormal round to 2^-149 (fp32) and 2^-133 (bf16), half of which is allowed
+# for each value beside the bar.
+@pytest.mark.parametrize("dtype,dim", [("bfloat16", 32), ("bfloat16", 128), ("float32", 32), ("float32", 64),
+                                       ("float32", 100)])
+@pytest.mark.parametrize("sizes,scale", [((1, 1, 1e-39, 1), None), ((1, 1, 1e-33, 1), None), ((1, 1, 1, 1e-36), None),
+                                         ((1, 1, 1, 1e-25), None), ((1e-36, 1e18, 1, 1), 1e17), ((1, 1, 1e-30, 1e-5), None),
+                                         ((1e-36, 1e-3, 1, 1), 1e30), ((1e8, 1e9, 1, 1), 1e-17), ((1, 1, 1, 1), 1e-20)])
+def test_small_operands_keep_their_bits(lm, dtype, dim, sizes, scale):
+    def change(*tensors):
+        for x, size in zip(tensors, sizes):
+            x *= np.float32(size)
+
+    (q, k, v, g), (out, dq, dk, dv), _ = run(lm, dtype, (1, 70, 2, 2, dim), True, 1, change, scale)
+    step = 2.0 ** (-150 if dtype == "float32" else -134)
+    for h in range(2):
+        o_ref, l_ref = ora.attention_np(q[0, h], k[0, h], v[0, h], scale=scale)
+        grads = ora.attention_backward_np(g[0, h], q[0, h], k[0, h], v[0, h], out[0, h], l_ref, scale=scale)
+        for name, got, exact in zip(("out", "dq", "dk", "dv"), (out, dq, dk, dv), (o_ref, *grads)):
+            allowed = BAR[dtype] * np.linalg.norm(exact) + step * exact.size ** 0.5
+            assert np.linalg.norm(got[0, h] - exact) <= allowed, (name, np.linalg.norm(got[0, h] - exact), allowed)
