@@ -575,6 +575,19 @@ Tile pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16, bool t
   return tiles[pick];
 }
 
+// The cheapest tile that launch_gathered_k has, for `groups` products.
+Tile gathered_k_tile(int64_t rows, int64_t cols, int64_t inner, int groups, bool bf16) {
+  if (forced_tile() >= 0) return (Tile)forced_tile();
+  Tile pick = TILE_L8D2;
+  if (!bf16) return pick;
+  double best = launch_cost(pick, tile_count(pick, rows, cols, groups), inner, true, true);
+  for (Tile t : {TILE_U, TILE_T}) {
+    const double cost = launch_cost(t, tile_count(t, rows, cols, groups), inner, true, true);
+    if (cost < 0.97 * best) best = cost, pick = t;
+  }
+  return pick;
+}
+
 Tile choose_tile(int64_t M, int64_t N, int64_t K, int64_t batch, bool bf16, bool ta) {
   if (forced_tile() >= 0) return (Tile)forced_tile();
   const int64_t cus = cu_count();
@@ -662,9 +675,13 @@ Tile grouped_tile(int64_t rows, int64_t inner, int64_t cols, int groups, bool bf
 // K chunks of a plain product (batch 1): the tile and the chunk count with the
 // lowest launch_cost over one chunk plus the partial sums' traffic ((2 s + 1)
 // x rows x cols fp32 values at 5 TB/s) and 4 us for the launch that adds them
-// up, if that is at least 15% below the product in one piece (the last kind
-// below: up to 5% above, where it measured 24 us against 28); below K = 512 the
-// second launch and its workspace cost the host more than the GPU gains.  Which products try:
+// up, if that is at least 15% below the product in one piece; below K = 512 the
+// second launch and its workspace cost the host more than the GPU gains.  For
+// the last kind below the bar is 5% above it: one piece of them measures 9 to
+// 16% more than its price (512 x 2048 over K = 4096: 27.5 and 31.4 us) and the
+// chunks, whose sums stay in the memory-side cache, up to 16% less (28 and 24);
+// of 210 such shapes that the rule splits, every one gained, by a fifth to
+// three quarters.  Which products try:
 //  * fp32 and thin outputs (<= 64 columns or rows): every one, on the small
 //    tiles; their tiles are long (fp32) or few (512 x 4096 x 512 fp32: 128 us
 //    in one piece, 32 in eight; a router's 8 logits; 30 x 2048 x 300 bf16:
@@ -1284,15 +1301,16 @@ int qutai_amd_gemm_grouped_k(const void* a, const void* b, void* out, const int6
   p.alpha = 1.0f;
   int64_t es = dtype == QA_BF16 ? 2 : 4;
   if ((p.lda * 256 * es) >= (1ll << 31) || (p.ldb * 256 * es) >= (1ll << 31)) return QA_EINVAL;
-  Tile tile = choose_tile(rows, cols, total_k / groups + 1, groups, dtype == QA_BF16, true);
   if (gather) {
     // row offsets into b are 32-bit byte offsets of one buffer descriptor
     if (source_rows < 0 || source_rows * cols * es >= (1ll << 31)) return QA_EINVAL;
     p.b_rows = gather;
     p.b_bytes = source_rows * cols * es;
+    const Tile tile = gathered_k_tile(rows, cols, total_k / groups + 1, groups, dtype == QA_BF16);
     return (int)(dtype == QA_F32 ? launch_gathered_k<true>(tile, p, stream)
                                  : launch_gathered_k<false>(tile, p, stream));
   }
+  const Tile tile = choose_tile(rows, cols, total_k / groups + 1, groups, dtype == QA_BF16, true);
   hipError_t err = dtype == QA_F32 ? launch_mma<true>(tile, true, false, p, stream)
                                    : launch_mma<false>(tile, true, false, p, stream);
   return (int)err;
