@@ -19,8 +19,8 @@ def owned(storage):
     hands to no one else: a leaf that receives it from the rule may keep it as
     its ``grad`` instead of copying it (the copy isolates storages a rule
     passes on to several tensors).  ``backward`` drops the mark from a storage
-    that does not go straight to a leaf: one that flows on through other rules
-    or is returned may be passed to several tensors later.  Returns the
+    that goes to another rule, which may pass it to several tensors; a rule that
+    itself runs a backward pass returns what its leaves received.  Returns the
     storage; None passes through."""
     if storage is not None:
         storage.owned_gradient = True
@@ -123,5 +123,6 @@ def backward(output, gradient, *, retain_graph=True, leaf_sink=None):
                     if isinstance(contribution, DeferredGradient):
                         fresh.add(parent)
                     gradients[parent] = contribution = _dense(contribution)
-                    take_owned(contribution)  # it goes on from here, to whatever tensors
+                    if parent.backward_rule is not None:
+                        take_owned(contribution)  # the rule may pass it on, to whatever tensors
     return leaves

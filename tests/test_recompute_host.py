@@ -67,9 +67,9 @@ def run_backward(output, seed):
 
 
 def test_a_gradient_that_goes_on_is_not_kept_by_a_leaf():
-    """A rule's own storage may be kept by the leaf it goes to straight away,
-    not after it went through another rule (which may pass it both ways) or out
-    of a checkpoint, whose stand-in leaves are not the graph's."""
+    """A rule's own storage may be kept by the leaf it goes to, out of a
+    checkpoint too, but not after it went through another rule, which may pass
+    it both ways (and a checkpoint's stand-in leaves are not the graph's)."""
     def product(x, y):
         out = Tensor(HostStorage(x.storage.values * y.storage.values), shape=x.shape)
         return grad.record(out, (x, y), lambda g: (grad.owned(HostStorage(g.values * y.storage.values)),
@@ -84,10 +84,8 @@ def test_a_gradient_that_goes_on_is_not_kept_by_a_leaf():
     x, z, w = leaf([1.0, 2.0]), leaf([3.0, 4.0]), leaf([5.0, 6.0])
     s = plus(x, z)
     for output in (product(s, w), recompute.checkpoint(lambda t: product(t, w), s, parameters=(w,))):
-        marks = kept(output)
-        assert not marks[x] and not marks[z]
+        assert kept(output) == {x: False, z: False, w: True}
     assert kept(product(x, w)) == {x: True, w: True}
-    assert not any(grad.take_owned(values) for values in run_backward(product(s, w), [1.0, 1.0]).values())
 
 
 def test_argument_and_declared_parameter_gradients_and_replay():
