@@ -52,7 +52,8 @@ int qutai_amd_device_arch(int device, char* name, size_t size);
  * runs on v_mfma_f32_32x32x16_bf16 with fp32 accumulation, an fp32 operand
  * being rounded to bf16 (nearest even) into `workspace` first (see
  * qutai_amd_gemm_workspace_size for when a workspace is needed and how
- * large); fp64 runs a SIMT kernel.  accumulate != 0 adds the old output before
+ * large; NULL where operands are used in place runs the product without K
+ * chunks); fp64 runs a SIMT kernel.  accumulate != 0 adds the old output before
  * the single rounding
  * to out_dtype.  inner == 0 writes zeros (or keeps out when accumulating).
  * Replaces: `cuda.gemm` (src/qutai/backends/cuda.py:305-362) and the kernels
@@ -88,11 +89,12 @@ int qutai_amd_gemm_static(const void* a, const void* b, void* out, int64_t rows,
 size_t qutai_amd_gemm_static_capacity(void);
 
 /* Bytes of workspace qutai_amd_gemm needs for these arguments with
- * 256-byte-aligned operands (0 when both operands are used in place).  An
- * operand is re-laid out into the workspace when its dtype differs from the
- * MFMA input type (fp32 into the bf16 path) or when its rows are not 16-byte
- * aligned (e.g. a 4097-wide row-major matrix): it then gets a zero-padded
- * pitch so every kernel load is a 16-byte vector load.  Helper of
+ * 256-byte-aligned operands (0 when both operands are used in place and K
+ * is not split into chunks, whose fp32 sums it holds).  An operand is
+ * re-laid out into the workspace when its dtype differs from the MFMA input
+ * type (fp32 into the bf16 path) or when its rows are not 16-byte aligned
+ * (e.g. a 4097-wide row-major matrix): it then gets a zero-padded pitch so
+ * every kernel load is a 16-byte vector load.  Helper of
  * qutai_amd_gemm with no reference counterpart (the reference narrows inside
  * its kernels, gemm.cu:21-24, and uses scalar loads). */
 size_t qutai_amd_gemm_workspace_size(int64_t rows, int64_t inner, int64_t cols, int64_t batch,

@@ -946,7 +946,8 @@ namespace qa {
 
 // A plain product.  With `spare`, K chunks whose partial sums do not fit beside
 // the operands' re-layouts are given up for the product in one piece (the
-// caller's workspace is fixed); without, a small workspace is an error.
+// caller's workspace is fixed, or there is none); without, a small workspace is
+// an error.
 int gemm_plain(const void* a, const void* b, void* out, int64_t rows, int64_t inner, int64_t cols,
                    int64_t batch, int64_t left_stride, int64_t right_stride, int transpose_left,
                    int transpose_right, int a_dtype, int b_dtype, int out_dtype, int accumulate,
@@ -1124,7 +1125,8 @@ int qutai_amd_gemm(const void* a, const void* b, void* out, int64_t rows, int64_
                    int transpose_right, int a_dtype, int b_dtype, int out_dtype, int accumulate,
                    int bf16_compute, void* workspace, size_t workspace_bytes, void* stream_) {
   return qa::gemm_plain(a, b, out, rows, inner, cols, batch, left_stride, right_stride, transpose_left, transpose_right,
-                    a_dtype, b_dtype, out_dtype, accumulate, bf16_compute, workspace, workspace_bytes, false, stream_);
+                    a_dtype, b_dtype, out_dtype, accumulate, bf16_compute, workspace, workspace ? workspace_bytes : 0,
+                    !workspace, stream_);
 }
 
 int qutai_amd_gemm_grouped(const void* a, const void* b, void* out, const int64_t* offsets, int groups,

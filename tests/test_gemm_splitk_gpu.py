@@ -105,3 +105,19 @@ def test_thin_outputs_split_by_themselves(amd, dtype, m, k, n, tb):
     rounded = download(amd.gemm(upload(a, dtype), upload(b, dtype), m, k, n, transpose_right=tb,
                                 out_dtype="bfloat16")).reshape(m, n)
     assert ora.rel_frobenius(rounded, exact) <= BF16_TOL
+
+
+@pytest.mark.parametrize("dtype,m,k,n", [("float32", 512, 640, 1024), ("float32", 300, 2048, 300),
+                                          ("bfloat16", 512, 4096, 1024), ("bfloat16", 32, 2048, 304)])
+def test_without_a_workspace_k_stays_whole(amd, dtype, m, k, n):
+    """Operands used in place need no workspace: where the plan has K chunks and
+    there is none for their sums, the product runs in one piece."""
+    runtime = amd.get_runtime()
+    code = 0 if dtype == "float32" else 5
+    shape = (m, k, n, 1, m * k, k * n, 0, 0, code, code, 0)
+    assert runtime.lib.qutai_amd_gemm_workspace_size(*shape) >= 2 * m * n * 4
+    a, b = normal(60, m * k), normal(61, k * n)
+    left, right, out = upload(a, dtype), upload(b, dtype), amd.full(m * n, 0.0, dtype="float32")
+    runtime.call("qutai_amd_gemm", left.ptr, right.ptr, out.ptr, *shape[:-1], 0, 0, 0, 0, 0)
+    exact = ora.gemm_f64(stored(a, dtype), stored(b, dtype), m, k, n)
+    assert ora.rel_frobenius(download(out).reshape(m, n), exact) <= FP32_TOL
