@@ -447,13 +447,19 @@ def _check_attention(q, k, v, batch, time, heads, kv_heads, dim):
         raise ValueError("q/k/v sizes do not match (batch, time, heads, dim)")
 
 
+def _on_matrix_cores(dtype, dim):
+    """Whether attention of this type and head dimension runs on the matrix
+    cores, for the launch counter (sequences of a few positions aside)."""
+    return dim % 8 == 0 if dtype == "bfloat16" else dim % 4 == 0 and dim <= 128
+
+
 def attention(q, k, v, batch, time, heads, kv_heads, dim, *, causal=True, layout=1, scale=None):
     """Attention forward (cuda_lm.attention, src/qutai/backends/cuda_lm.py:229-275):
     (out, lse float32).  bf16 q/k/v with head dimension 64 run the fused MFMA
     kernel; other head dimensions (<= 256) and float32 storage run the MFMA
-    kernels that keep fp32 values in bf16 parts, rows that are not 16-byte
-    aligned (and fp32 above 128) the one-wave-per-row kernel, the reference's
-    own fallback shape.
+    kernels that keep fp32 values in bf16 parts; rows that are not 16-byte
+    aligned, fp32 above 128 and sequences of a few positions the
+    one-wave-per-row kernel, the reference's own fallback shape.
     layout 1 is the lm layout [batch][time][heads][dim], layout 0 the nn
     layout [batch][heads][time][dim].  The score matrix is never stored."""
     _check_attention(q, k, v, batch, time, heads, kv_heads, dim)
@@ -463,7 +469,7 @@ def attention(q, k, v, batch, time, heads, kv_heads, dim, *, causal=True, layout
     if q.size:
         out.runtime.call("qutai_amd_attention_fwd", q.ptr, k.ptr, v.ptr, out.ptr, lse.ptr, batch, heads, kv_heads,
                          time, dim, code(q.dtype), layout, float(scale), int(bool(causal)),
-                         mfma=q.dtype == "bfloat16" and dim == 64)
+                         mfma=_on_matrix_cores(q.dtype, dim))
     return out, lse
 
 
@@ -552,7 +558,7 @@ def attention_backward(gradient, q, k, v, out, lse, batch, time, heads, kv_heads
         workspace = AMDStorage((need + 3) // 4, "float32") if need else None
         runtime.call("qutai_amd_attention_bwd", gradient.ptr, q.ptr, k.ptr, v.ptr, out.ptr, lse.ptr, dq.ptr, dk.ptr,
                      dv.ptr, delta.ptr, workspace.ptr if workspace else None, need, batch, heads, kv_heads, time, dim,
-                     code(q.dtype), layout, float(scale), int(bool(causal)), mfma=q.dtype == "bfloat16" and dim == 64)
+                     code(q.dtype), layout, float(scale), int(bool(causal)), mfma=_on_matrix_cores(q.dtype, dim))
     return dq, dk, dv
 
 

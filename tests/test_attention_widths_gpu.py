@@ -169,3 +169,14 @@ def test_small_operands_keep_their_bits(lm, dtype, dim, sizes, scale):
         for name, got, exact in zip(("out", "dq", "dk", "dv"), (out, dq, dk, dv), (o_ref, *grads)):
             allowed = BAR[dtype] * np.linalg.norm(exact) + step * exact.size ** 0.5
             assert np.linalg.norm(got[0, h] - exact) <= allowed, (name, np.linalg.norm(got[0, h] - exact), allowed)
+
+
+@pytest.mark.parametrize("dtype,dim,counted", [("bfloat16", 64, True), ("bfloat16", 200, True), ("float32", 100, True),
+                                               ("float32", 132, False), ("bfloat16", 36, False)])
+def test_matrix_core_launches_are_counted(lm, dtype, dim, counted):
+    from qutai_amd.backends import amd
+
+    runtime = amd.get_runtime()
+    before = runtime.mfma_launches
+    run(lm, dtype, (1, 40, 2, 1, dim), True, 1)
+    assert runtime.mfma_launches - before == (2 if counted else 0)

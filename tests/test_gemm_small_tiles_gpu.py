@@ -1,7 +1,8 @@
 """The eight-wave 128x128 (X), 128x64 (Y) and 64x64 (Z) tiles: forced, they give
 the bits of the 256x256 tile (every tile sums K in the same order), and their
-copies, with the 16-wide K stages in which fp32 operands are read, stay inside
-the operands (the CPU model of the kernels' addressing)."""
+copies stay inside the operands (the CPU model of the kernels' addressing: the
+ring that bf16 and the fp32 MFMA read, and the 16-wide K stages, some past K, in
+which the fp32 parts are read)."""
 import numpy as np
 import pytest
 
