@@ -45,6 +45,12 @@ void launch_pass(Pass pass, const AttnGenArgs& a, unsigned blocks, hipStream_t s
 // need more registers than a wave has (three parts of q and dO).
 bool mma_fits(int dtype, int64_t dim) { return dtype == BF16 ? dim % 8 == 0 && dim <= 256 : dim % 4 == 0 && dim <= 128; }
 
+// Whether 64 rows of every operand lie within the 2 GiB of a buffer descriptor,
+// beyond which the kernels' loads read zeros (rows of 8 million fp32 values).
+bool mma_spans(const AttnGenArgs& a, int dtype) {
+  return 64 * std::max(a.qt, a.kt) * (dtype == F32 ? 4 : 2) <= 0x7ffffff0;
+}
+
 // A scale of the scores with which the factors that take the parts' scaling
 // back (2^-48 at most) keep their bits: any in earnest use.
 bool mma_scale(double scale) { return scale >= 0x1p-50; }
@@ -124,7 +130,7 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
   a.causal = causal ? 1 : 0;
   const int64_t rows = batch * heads * time;
   if ((rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
-  if (mma_fits(dtype, dim) && mma_scale(scale) && aligned16({q, k, v, out}) &&
+  if (mma_fits(dtype, dim) && mma_scale(scale) && mma_spans(a, dtype) && aligned16({q, k, v, out}) &&
       !few_positions(dtype, batch, heads, time, dim, false))
     return (int)launch_mma(FORWARD, dtype, a, batch * heads * ((time + OWNED - 1) / OWNED), stream);
   return (int)launch_rows(attention_fwd_rows<bf16_t>, attention_fwd_rows<float>, dtype, a, rows, stream);
@@ -161,7 +167,8 @@ int attention_general_bwd(const void* grad, const void* q, const void* k, const 
   const int64_t q_rows = batch * heads * time, k_rows = batch * kv_heads * time;
   if ((q_rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
   // the q pass writes delta, which the kv pass reads
-  if (!mma_fits(dtype, dim) || !mma_scale(scale) || !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
+  if (!mma_fits(dtype, dim) || !mma_scale(scale) || !mma_spans(a, dtype) ||
+      !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
       few_positions(dtype, batch, heads, time, dim, true)) {
     const hipError_t e =
         launch_rows(attention_bwd_q_rows<bf16_t>, attention_bwd_q_rows<float>, dtype, a, q_rows, stream);

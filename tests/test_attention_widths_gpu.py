@@ -180,3 +180,17 @@ def test_matrix_core_launches_are_counted(lm, dtype, dim, counted):
     before = runtime.mfma_launches
     run(lm, dtype, (1, 40, 2, 1, dim), True, 1)
     assert runtime.mfma_launches - before == (2 if counted else 0)
+
+
+def test_rows_beyond_a_descriptor(lm):
+    """Positions 87 MB apart: those from the 25th on of a block of 32 lie beyond
+    the 2 GiB that a buffer descriptor spans.  Equal keys average the values, all
+    ones; one that read as zeros would show."""
+    from qutai_amd.backends import amd
+
+    time, heads, dim = 48, 170000, 128
+    ones = amd.full(time * heads * dim, 1.0, dtype="float32")
+    out, _ = lm.attention(ones, ones, ones, 1, time, heads, heads, dim, causal=False)
+    means = download(amd.mean(out, (time, heads * dim), 1))
+    del out
+    assert np.abs(means - 1).max() <= 1e-3
