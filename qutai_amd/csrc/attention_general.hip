@@ -91,15 +91,23 @@ constexpr int64_t OWNED = 128;  // queries or keys of a workgroup
 
 // Whether a call takes one wave per row although the matrix kernels could hold
 // it: the tiles of a sequence of a few positions are mostly empty, and sums of
-// one or two terms round best on their own.  Measured with 16000 heads (us;
-// rows, tiles): forward bf16 D 128, T 6 103 and 178, T 8 191 and 180; bf16 D 32,
-// T 6 72 and 75; fp32 D 64, T 8 128 and 148; backward bf16 D 128 with a quarter of
-// the kv heads, T 2 45 and 723, T 12 618 and 739; bf16 D 32, T 6 153 and 168, T 8
-// 279 and 168; fp32 D 32, T 8 270 and 312.  Grids of fewer heads than the GPU
-// holds at once take the tiles earlier (32 heads of 128, bf16: forward, T 3, 10 and
-// 7.6; backward, T 4, 20 and 22, T 5 24 and 22).
-bool few_positions(int dtype, int64_t batch, int64_t heads, int64_t time, int64_t dim, bool backward) {
-  const int64_t most = dim > 32 ? (backward ? 12 : 8) : backward && dtype == F32 ? 8 : 6;
+// one or two terms round best on their own.  Measured with 8000 and 16000 heads
+// (us; rows, tiles), the lines lie at the crossings: forward bf16 D 32, T 6 72
+// and 75; bf16 D 128, T 6 103 and 178, T 8 191 and 180; bf16 D 136, T 10 154 and
+// 209, T 13 236 and 209; fp32 D 64, T 8 128 and 148, T 13 121 and 80 (8000); fp32
+// D 96, T 10 116 and 181, T 13 179 and 182; fp32 D 128, T 13 181 and 218, T 16 357
+// and 216.  Backward bf16 D 32, T 6 153 and 168, T 8 279 and 168; fp32 D 32, T 8
+// 270 and 312; bf16 D 128, T 2 45 and 723, T 13 390 and 469 (8000); fp32 D 64,
+// T 13 251 and 354; fp32 D 128, T 13 433 and 1021, T 20 885 and 1061.  Grids of
+// fewer heads than the GPU holds at once take the tiles earlier (32 heads of
+// 128, bf16: forward, T 3, 10 and 7.6; backward, T 4, 20 and 22, T 5 24 and 22).
+bool few_positions(int dtype, int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim,
+                   bool backward) {
+  const bool f32 = dtype == F32;
+  int64_t most;
+  if (dim <= 32) most = f32 ? (backward ? 8 : 7) : 6;
+  else if (backward) most = f32 && dim > 96 && heads == kv_heads ? 20 : 13;
+  else most = f32 ? (dim <= 64 ? 8 : 13) : dim <= 128 ? 8 : 10;
   return time <= (backward ? 4 : 2) || (time <= most && batch * heads >= 2 * cu_count());
 }
 
@@ -131,7 +139,7 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
   const int64_t rows = batch * heads * time;
   if ((rows + GEN_WAVES - 1) / GEN_WAVES > 0x7fffffff) return QA_EINVAL;
   if (mma_fits(dtype, dim) && mma_scale(scale) && mma_spans(a, dtype) && aligned16({q, k, v, out}) &&
-      !few_positions(dtype, batch, heads, time, dim, false))
+      !few_positions(dtype, batch, heads, kv_heads, time, dim, false))
     return (int)launch_mma(FORWARD, dtype, a, batch * heads * ((time + OWNED - 1) / OWNED), stream);
   return (int)launch_rows(attention_fwd_rows<bf16_t>, attention_fwd_rows<float>, dtype, a, rows, stream);
 }
@@ -139,7 +147,7 @@ int attention_general_fwd(const void* q, const void* k, const void* v, void* out
 size_t attention_general_workspace(int64_t batch, int64_t heads, int64_t kv_heads, int64_t time, int64_t dim,
                                    int dtype) {
   if ((dtype != BF16 && dtype != F32) || dim <= 0 || batch < 0 || time < 0 || !mma_fits(dtype, dim)) return 0;
-  if (few_positions(dtype, batch, heads, time, dim, true)) return 0;
+  if (few_positions(dtype, batch, heads, kv_heads, time, dim, true)) return 0;
   return split_bytes(batch, heads, kv_heads, time, dim);
 }
 
@@ -169,7 +177,7 @@ int attention_general_bwd(const void* grad, const void* q, const void* k, const 
   // the q pass writes delta, which the kv pass reads
   if (!mma_fits(dtype, dim) || !mma_scale(scale) || !mma_spans(a, dtype) ||
       !aligned16({grad, q, k, v, out, dq, dk, dv}) ||
-      few_positions(dtype, batch, heads, time, dim, true)) {
+      few_positions(dtype, batch, heads, kv_heads, time, dim, true)) {
     const hipError_t e =
         launch_rows(attention_bwd_q_rows<bf16_t>, attention_bwd_q_rows<float>, dtype, a, q_rows, stream);
     if (e != hipSuccess) return (int)e;

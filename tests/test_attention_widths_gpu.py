@@ -119,8 +119,9 @@ def test_a_query_of_one_key_has_no_gradient(lm, dims):
     assert not dq[:, :, 0].any() and out[:, :, 0].any()
 
 
-@pytest.mark.parametrize("dtype,dim", [("bfloat16", 32), ("bfloat16", 128), ("float32", 32), ("float32", 64)])
-@pytest.mark.parametrize("time", [1, 2, 3, 6, 7, 8, 9, 12, 13])
+@pytest.mark.parametrize("dtype,dim", [("bfloat16", 32), ("bfloat16", 128), ("bfloat16", 136), ("float32", 32),
+                                       ("float32", 64), ("float32", 100)])
+@pytest.mark.parametrize("time", [1, 2, 3, 6, 7, 8, 9, 10, 11, 13, 14, 20, 21])
 @pytest.mark.parametrize("heads", [2, 512])
 def test_short_sequences(lm, dtype, dim, time, heads):
     """Both sides of the lines between one wave per row and tiles, for grids that
