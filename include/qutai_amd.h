@@ -384,16 +384,19 @@ int qutai_amd_combine(const void* expert_out, const float* weights, const int64_
  *   out = softmax(scale * Q K^T [+ causal mask]) V  per (batch, head),
  * without materialising the time x time scores.  dtype QA_BF16 or QA_F32 for
  * q, k, v and out; head dimension `dim` <= 256.  bf16 with dim = 64 runs the
- * fused MFMA kernel (16-byte aligned pointers required); every other case the
- * one-wave-per-row kernel of the reference's general path.  layout 0: q/k/v/out
- * are [batch][heads][time][dim] (the nn layout); layout 1:
- * [batch][time][heads][dim] (the lm layout, head-interleaved).  kv_heads divides heads (grouped-query
- * attention: head h reads kv head h / (heads / kv_heads)).  lse (optional,
+ * fused MFMA kernel (16-byte aligned pointers required); bf16 with other
+ * multiples of 8 and fp32 with multiples of 4 up to 128, 16-byte aligned, MFMA
+ * kernels that keep fp32 values in three bf16 parts; every other case, and
+ * sequences of a few positions, the one-wave-per-row kernel of the reference's
+ * general path.  layout 0: q/k/v/out are [batch][heads][time][dim] (the nn
+ * layout); layout 1: [batch][time][heads][dim] (the lm layout,
+ * head-interleaved).  kv_heads divides heads (grouped-query attention: head h
+ * reads kv head h / (heads / kv_heads)).  lse (optional,
  * fp32) receives the natural-log sum of exponentials, laid out like q without
  * the last axis: [batch][heads][time] (layout 0), [batch][time][heads]
  * (layout 1, the reference's lse layout).  The normaliser sums fp32
- * probabilities; the value product takes them rounded to bf16, as in the
- * reference kernel.  Replaces `lm_attention_bf16_d64` and the general
+ * probabilities; the value product takes them as they are, or (bf16 with dim =
+ * 64) rounded to bf16, as in the reference kernel.  Replaces `lm_attention_bf16_d64` and the general
  * `lm_attention` (src/qutai/backends/cuda/lm.cu:91-157, :65-87, driven by
  * `cuda_lm.attention`, src/qutai/backends/cuda_lm.py:229-252) and the
  * S = Q K^T / softmax / P V sequence of nn attention
@@ -406,7 +409,8 @@ int qutai_amd_attention_fwd(const void* q, const void* k, const void* v, void* o
  * positions whose last `length` are the new ones: query i sees the first
  * total - length + i + 1 keys.  q and out are [batch][length][heads][dim], k
  * and v [batch][heads][total][dim], all of `dtype` (QA_BF16 with dim % 8 == 0,
- * QA_F32 with dim % 4 == 0; dim <= 256) and 16-byte aligned; total <= 12000.
+ * QA_F32 with dim % 4 == 0; dim <= 256) and 16-byte aligned; total <= 12000,
+ * batch x heads x length below 2^22.
  * Scores, probabilities and sums are fp32.  Replaces the Q K^T / softmax / P V
  * sequence of the cache path (src/qutai/nn/layers.py:345-355). */
 int qutai_amd_attention_cached(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t heads,
@@ -414,8 +418,9 @@ int qutai_amd_attention_cached(const void* q, const void* k, const void* v, void
 
 /* A key and a value cache extended in one launch: out[r] = past[r] followed by
  * new[r] for each of `rows` (batch, head) rows of past_bytes and new_bytes, both
- * multiples of 16, all pointers 16-byte aligned; out does not overlap the
- * inputs.  Replaces the concatenations of src/qutai/nn/cache.py:5-29. */
+ * multiples of 16, all pointers 16-byte aligned (NULL for empty parts); out
+ * does not overlap the inputs; rows x 16 KiB segments of an output row below
+ * 2^23.  Replaces the concatenations of src/qutai/nn/cache.py:5-29. */
 int qutai_amd_cache_join(const void* past_k, const void* past_v, const void* new_k, const void* new_v, void* out_k,
                          void* out_v, int64_t rows, int64_t past_bytes, int64_t new_bytes, void* stream);
 
